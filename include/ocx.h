@@ -243,9 +243,9 @@ typedef struct ocx_domain {
 
 typedef struct ocx_batch ocx_batch;
 
-/* rows_per_chunk: rows one wavefront marches (0: 64); waves_per_group: wavefronts per workgroup, the tracers of one
- * layer (0: 2, at most 4); groups_per_cu: resident workgroups per compute unit of the persistent grid (0: 4).  Copies
- * the domain table to the device (synchronous). */
+/* rows_per_chunk: rows one wavefront marches (0: 2 .. 64, by the wavefronts the call gives); waves_per_group:
+ * wavefronts per workgroup, the tracers of one layer (0: 2, at most 4); groups_per_cu: resident workgroups per compute
+ * unit of the persistent grid (0: 4).  Copies the domain table to the device (synchronous). */
 int ocx_batch_create(const ocx_domain* domains, int ndomains, int rows_per_chunk, int waves_per_group,
                      int groups_per_cu, ocx_batch** out);
 int ocx_batch_step(ocx_batch* batch, int parity, void* stream);

@@ -102,13 +102,34 @@ size_t fct_layout(void* base, int nt, int nz, int ny, int nx, FctWs* w) {
 
 // launch shape of the single-domain calls (ocx_set_tuning): rows per chunk, waves per workgroup (0: default)
 std::atomic<int> g_rch{0}, g_wpb{0};
-constexpr int DEFAULT_RCH = 64;
+constexpr int MAX_RCH = 64;
 constexpr int DEFAULT_WPB = 1;    // one tracer of a layer per workgroup (measured best at 1024 x 1024 x 50 x 10)
 constexpr int DEFAULT_BATCH_WPB = 2;    // the persistent batch's default (measured best on the 64-domain batch)
 
-int rows_per_chunk() {
+// Rows per chunk by the wavefronts a launch gives.  A wavefront marches its chunk row by row, a serial chain of about
+// 2 us per row and stage, so while the launch leaves the chip idle the time is that chain's and short chunks win; once
+// it is full, every chunk's halo rows and first face cost about one row more.  waves(r) = wavefronts with chunks of r
+// rows.  Measured (us per FP64 step, chunks of 64 -> chosen): 96 x 80 x 8 x 2 tracers 484 -> 45 (2 rows; 4 rows 51),
+// 128 x 128 x 20 x 2 477 -> 98 (4; 2 rows 110), 198 x 159 x 50 x 1 491 -> 174 (4), 352 x 560 x 50 x 2 1631 -> 1407
+// (16; 32 rows 1466, 8 rows 1454), 384 x 384 x 50 x 10 5073 -> 4982 (32; 16 rows 5084), 701 x 523 x 30 x 10 7433 ->
+// 7291 (32); at 1024 x 1024 x 50 x 10 chunks of 64 rows stay the best (33.6 ms, 32 rows 33.8).  So: 64 rows while they
+// give 65536 wavefronts (16 to each of the 4096 slots of 1024 SIMDs), else the longest chunk of 32 .. 4 rows that
+// gives 16384, and 2 rows where even chunks of 4 leave SIMDs without a wavefront.
+template <class Waves>
+int auto_rows(Waves&& waves) {
+    if (waves(MAX_RCH) >= 65536) return MAX_RCH;
+    int r = MAX_RCH / 2;
+    while (r > 4 && waves(r) < 16384) r /= 2;
+    return r == 4 && waves(r) < 1024 ? 2 : r;
+}
+// wavefronts of one domain's stage launch with chunks of r rows
+long long march_waves(int nt, int nz, int ny, int nx, int r) {
+    return (long long)((nx + ocx::MS - 1) / ocx::MS) * ((ny + r - 1) / r) * nt * nz;
+}
+
+int rows_per_chunk(int nt, int nz, int ny, int nx) {
     const int r = g_rch.load();
-    return r > 0 ? r : DEFAULT_RCH;
+    return r > 0 ? r : auto_rows([&](int rr) { return march_waves(nt, nz, ny, nx, rr); });
 }
 
 // waves per workgroup = tracers per group: the tracers split into groups of at most `cap` (<= MAXW), as even as
@@ -278,7 +299,7 @@ int advect_fct_impl(const double* C, const double* V0, const double* V1, const d
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool js = flags & WENO_JS, unlim = flags & UNLIMITED;
     const int fi = fx_i ? flux_face_i : -1;
-    const int rch = rows_per_chunk();
+    const int rch = rows_per_chunk(nt, nz, ny, nx);
     if ((long long)((nx + LS - 1) / LS) * ((ny + rch - 1) / rch) * nt * nz >= (1LL << 31))
         return fail(OCX_E_ARG, "shape (nt=%d, nz=%d, ny=%d, nx=%d) too large for one launch", nt, nz, ny, nx);
     MarchArgs a{};
@@ -830,9 +851,18 @@ int ocx_batch_create(const ocx_domain* domains, int ndomains, int rows_per_chunk
     if (rows_per_chunk < 0 || waves_per_group < 0 || waves_per_group > MAXW || groups_per_cu < 0)
         return fail(OCX_E_ARG, "bad tuning (rows_per_chunk=%d, waves_per_group=%d, groups_per_cu=%d)",
                     rows_per_chunk, waves_per_group, groups_per_cu);
-    const int rch = rows_per_chunk > 0 ? rows_per_chunk : DEFAULT_RCH;
     int maxnt = 1;
-    for (int d = 0; d < ndomains; ++d) maxnt = std::max(maxnt, domains[d].nt);
+    for (int d = 0; d < ndomains; ++d) {
+        OCX_TRY(check_shape(domains[d].nt, domains[d].nz, domains[d].ny, domains[d].nx));
+        maxnt = std::max(maxnt, domains[d].nt);
+    }
+    // rows per chunk by the wavefronts of all members together, which share the launch
+    const int rch = rows_per_chunk > 0 ? rows_per_chunk : auto_rows([&](int r) {
+        long long w = 0;
+        for (int d = 0; d < ndomains; ++d)
+            w += march_waves(domains[d].nt, domains[d].nz, domains[d].ny, domains[d].nx, r);
+        return w;
+    });
     // two tracers per workgroup unless asked otherwise (the 64-domain batch measured 149.5 ms per step with two,
     // 150.7 with one)
     const int wg = waves_per_group > 0 ? waves_per_group : DEFAULT_BATCH_WPB;
@@ -841,7 +871,6 @@ int ocx_batch_create(const ocx_domain* domains, int ndomains, int rows_per_chunk
     std::vector<long long> pm(ndomains + 1, 0), pl(ndomains + 1, 0);
     for (int d = 0; d < ndomains; ++d) {
         const ocx_domain& D = domains[d];
-        OCX_TRY(check_shape(D.nt, D.nz, D.ny, D.nx));
         if (!D.C || !D.C_out || !D.V0 || !D.V1 || !D.Qx || !D.Qy || !D.ok || !D.workspace)
             return fail(OCX_E_ARG, "domain %d: a required pointer is NULL", d);
         if (D.C == D.C_out) return fail(OCX_E_ARG, "domain %d: C and C_out alias", d);
