@@ -53,6 +53,29 @@ long long rk_blocks(int nt, int ny, int nx, int tx) {
     return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * nt;
 }
 
+// Layers that one block of the layer-marching kernel marches.  A block's start (its window, its first tile, its bottom
+// face) costs about 1.5 layers, and a launch takes as many rounds as its blocks need on the resident slots (3 blocks a
+// compute unit with the WENO faces, 4 with the cheaper ones), so the column is cut into the number of pieces that makes
+// rounds x (layers + 1.5) the least, if that is a tenth less than for the whole column; pieces beyond 64, or launches
+// beyond 2^24 blocks, never gain.  Whole column -> cut (us per step): RK3 128 x 128 x 20 x 2 tracers 285 -> 112 (4
+// layers; 2 layers 114, 10 layers 156), 198 x 159 x 50 x 1 717 -> 221 (5); 352 x 560 x 50 x 4 stays whole (3281,
+// pieces of 25 layers 3348), as does 1024 x 1024 x 50 x 10; pc with UP3 faces 128 x 128 x 20 x 2 110 -> 38 (3; 2 layers 44, 5 layers 43), 300 x 250 x 30 x 4 346 -> 289 (10).
+int rk_layers(long long tiles, int nz, int blocks_per_cu) {
+    const long long slots = 256LL * blocks_per_cu;
+    int best = nz;
+    double least = 0.0;
+    for (int c = 1; c <= std::min(nz, 64) && (c == 1 || tiles * c <= (1LL << 24)); ++c) {
+        const int kl = (nz + c - 1) / c;
+        const long long nb = tiles * ((nz + kl - 1) / kl);
+        const double cost = (double)((nb + slots - 1) / slots) * (kl + 1.5);
+        if (c == 1 || cost < least) {
+            least = c == 1 ? 0.9 * cost : cost;
+            best = kl;
+        }
+    }
+    return best;
+}
+
 int check_shape(int nt, int nz, int ny, int nx) {
     if (nt < 1 || nz < 1 || ny < 1 || nx < 1)
         return fail(OCX_E_ARG, "shape (nt=%d, nz=%d, ny=%d, nx=%d) must be positive", nt, nz, ny, nx);
@@ -201,14 +224,19 @@ struct RkArgs {
     unsigned flags;
 };
 
-// k_rk_stage runs one block per (tile, tracer) on a 1-D grid; the host checks the block count fits it.
+// k_rk_stage runs one block per (tile, tracer, piece of the column) on a 1-D grid; the host checks that the whole
+// columns' count fits it.
 template <int STAGE, int SCH, bool VERT>
 void rk_launch(const RkArgs& a, dim3, hipStream_t s) {
     constexpr int tx = rk_tx<SCH>(), ty = 256 / tx;
-    const long long nb = rk_blocks(a.nt, a.ny, a.nx, tx);
-    ocx::k_rk_stage<STAGE, SCH, VERT, tx, ty><<<dim3((unsigned)nb), dim3(64, 4), 0, s>>>(
-        a.cin, a.C, a.ext, a.V0, a.V1, a.Qx, a.Qy, a.Fz, a.ok, a.q, a.cout, a.fxs, a.fi, a.nt, a.nz, a.ny, a.nx, a.dt,
-        a.flags);
+    const long long tiles = rk_blocks(a.nt, a.ny, a.nx, tx);
+    const int kl = rk_layers(tiles, a.nz, SCH <= ocx::SCH_Z ? 3 : 4);
+    const long long nb = tiles * ((a.nz + kl - 1) / kl);
+    // the cut kernel is one of its own: its extra face costs the uncut one 6 % (registers), so a cut has to gain 10 %
+    auto* kern = kl < a.nz ? ocx::k_rk_stage<STAGE, SCH, VERT, true, tx, ty>
+                           : ocx::k_rk_stage<STAGE, SCH, VERT, false, tx, ty>;
+    kern<<<dim3((unsigned)nb), dim3(64, 4), 0, s>>>(a.cin, a.C, a.ext, a.V0, a.V1, a.Qx, a.Qy, a.Fz, a.ok, a.q, a.cout,
+                                                    a.fxs, a.fi, a.nt, a.nz, a.ny, a.nx, kl, a.dt, a.flags);
 }
 
 // One RK3 or 'pc' stage (STAGE 0: the RHS only) with the scheme's faces; UP3 / UP1 / centred always form the z
@@ -216,12 +244,20 @@ void rk_launch(const RkArgs& a, dim3, hipStream_t s) {
 template <int STAGE>
 void rk_stage(const RkArgs& a, int sch, bool vert, dim3 grid, hipStream_t s) {
     using namespace ocx;
-    switch (sch) {
-        case SCH_C6: rk_launch<STAGE, SCH_C6, true>(a, grid, s); break;
-        case SCH_UP3: rk_launch<STAGE, SCH_UP3, true>(a, grid, s); break;
-        case SCH_UP1: rk_launch<STAGE, SCH_UP1, true>(a, grid, s); break;
-        case SCH_JS: vert ? rk_launch<STAGE, SCH_JS, true>(a, grid, s) : rk_launch<STAGE, SCH_JS, false>(a, grid, s); break;
-        default: vert ? rk_launch<STAGE, SCH_Z, true>(a, grid, s) : rk_launch<STAGE, SCH_Z, false>(a, grid, s);
+    if constexpr (STAGE == 4) {
+        rk_launch<STAGE, SCH_C6, true>(a, grid, s);      // the pc predictor has centred faces
+    } else {
+        switch (sch) {
+            case SCH_C6:
+                if constexpr (STAGE == 0) rk_launch<STAGE, SCH_C6, true>(a, grid, s);   // only the RHS takes them
+                break;
+            case SCH_UP3: rk_launch<STAGE, SCH_UP3, true>(a, grid, s); break;
+            case SCH_UP1: rk_launch<STAGE, SCH_UP1, true>(a, grid, s); break;
+            case SCH_JS:
+                vert ? rk_launch<STAGE, SCH_JS, true>(a, grid, s) : rk_launch<STAGE, SCH_JS, false>(a, grid, s);
+                break;
+            default: vert ? rk_launch<STAGE, SCH_Z, true>(a, grid, s) : rk_launch<STAGE, SCH_Z, false>(a, grid, s);
+        }
     }
 }
 

@@ -464,18 +464,19 @@ __device__ __forceinline__ double zface_w(const double* w, const bool* b, double
 #define OCX_RK_WAVES 3
 #endif
 
-template <int STAGE, int SCH, bool VERT, int TX, int TY>
+template <int STAGE, int SCH, bool VERT, bool CUT, int TX, int TY>
 __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(OCX_RK_WAVES))) void k_rk_stage(const double* __restrict__ cin, const double* __restrict__ C,
                                                      const double* __restrict__ ext, const double* __restrict__ V0,
                                                      const double* __restrict__ V1, const double* __restrict__ Qx,
                                                      const double* __restrict__ Qy, const double* __restrict__ Fz,
                                                      const uint8_t* __restrict__ ok, double* __restrict__ q,
                                                      double* __restrict__ cout, double* __restrict__ fxs,
-                                                     int flux_face_i, int nt, int n, int ny, int nx, double dt,
+                                                     int flux_face_i, int nt, int n, int ny, int nx, int kl, double dt,
                                                      unsigned flags) {
-    // One block marches one tile of one tracer up its layers (1-D grid of nt * gx * gy blocks, XCD-contiguous):
-    // each layer's x and y faces go through the LDS tile; each thread keeps its column's window c[k-2 .. k+3] in
-    // registers and forms the z face between layers k and k+1 once, carrying it as the next layer's bottom face.
+    // One block marches one tile of one tracer up its layers - all of them, or with CUT kl of them (1-D grid of
+    // nt * gx * gy * ceil(n / kl) blocks, XCD-contiguous): each layer's x and y faces go through the LDS tile; each thread keeps its column's window
+    // c[k-2 .. k+3] in registers and forms the z face between layers k and k+1 once, carrying it as the next layer's
+    // bottom face.
     constexpr bool ZF = VERT || SCH >= SCH_UP3;
     constexpr int H = 3, LX = TX + 2 * H, LY = TY + 2 * H;
     __shared__ double sc[LY * LX];
@@ -490,13 +491,14 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(OCX_RK_W
     const int tid = threadIdx.y * 64 + threadIdx.x;
     const int ty = TX == 64 ? (int)threadIdx.y : tid / TX, tx = TX == 64 ? (int)threadIdx.x : tid - ty * TX;
     const int gx = (nx + TX - 1) / TX, gy = (ny + TY - 1) / TY;
-    const long long nb = (long long)gx * gy * nt;
     // tracer fastest: the nt blocks of a tile run together on one XCD and share its per-layer fields through L2
-    long long L = xcd_logical((long long)blockIdx.x, nb);
+    long long L = xcd_logical((long long)blockIdx.x, (long long)gridDim.x);
     const int t = (int)(L % nt);
     L /= nt;
     const int bx = (int)(L % gx);
-    const int by = (int)(L / gx);
+    L /= gx;
+    const int by = CUT ? (int)(L % gy) : (int)L;
+    const int k0 = CUT ? (int)(L / gy) * kl : 0, k1 = CUT ? min(k0 + kl, n) : n;
     const int i0 = bx * TX, j0 = by * TY;
     const size_t plane = (size_t)ny * nx;
     const int j = j0 + ty, i = i0 + tx;
@@ -515,16 +517,35 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(OCX_RK_W
     };
     // bit m: w[m] is 0 or of magnitude in [2^-400, 2^100]
     unsigned wfast = 0;
-    if constexpr (ZF) {
-#pragma unroll
-        for (int m = 0; m < 6; ++m) {
-            wload(m, m - 2);
-            if constexpr (WENO) wfast |= (unsigned)fast_value(w[m]) << m;
-        }
-    }
-    // the bottom face of layer 0: 0 for WENO, Fz[0] * 0 for the rhs_numpy faces
+    // the bottom face of layer k0: at the bed 0 for WENO, Fz[0] * 0 for the rhs_numpy faces; above it interface k0's
+    // face, which the block below forms too (the same expression on the same values)
     double fb = 0.0;
     if constexpr (SCH >= SCH_UP3) fb = cell ? Fz[xc] * 0.0 : 0.0;
+    if constexpr (ZF) {
+        const int kw = CUT && k0 > 0 ? k0 - 1 : k0;
+#pragma unroll
+        for (int m = 0; m < 6; ++m) {
+            wload(m, kw + m - 2);
+            if constexpr (WENO) wfast |= (unsigned)fast_value(w[m]) << m;
+        }
+        if (CUT && k0 > 0) {
+            const double qz = cell ? Fz[(size_t)k0 * plane + xc] : 0.0;
+            fb = 0.0;
+            if (cell) {
+                if constexpr (SCH >= SCH_UP3)
+                    fb = qz * zface_w<SCH>(w, b, qz);
+                else if (qz != 0.0)
+                    fb = zface_w<SCH>(w, b, qz, wfast == 0x3fu);
+            }
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                w[m] = w[m + 1];
+                b[m] = b[m + 1];
+            }
+            wload(5, k0 + 3);
+            if constexpr (WENO) wfast = (wfast >> 1) | ((unsigned)fast_value(w[5]) << 5);
+        }
+    }
     // the tile of layer k (with its halo) is fetched into registers one layer ahead and stored to LDS at the top of
     // the layer's iteration, so its loads are in flight while the previous layer's faces are formed
     constexpr int NT = TX * TY, NL = (LY * LX + NT - 1) / NT;
@@ -555,13 +576,13 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(OCX_RK_W
         tile_face_q_waves<TX, TY>(qn4, Qx + (size_t)kk * ny * (nx + 1), Qy + (size_t)kk * (ny + 1) * nx, i0, j0, ny,
                                   nx);
     };
-    fetch(0);
-    fetch_q(0);
+    fetch(k0);
+    fetch_q(k0);
     if constexpr (WENO) {
         if (tid < 2) sbad[tid] = 0;
         __syncthreads();
     }
-    for (int k = 0; k < n; ++k) {
+    for (int k = k0; k < k1; ++k) {
         const int p = t * n + k;
         const size_t pc = (size_t)p * plane, kc = (size_t)k * plane;
         // no barrier needed before the store: the tile (sc, so) was last read by the previous layer's face phase,
@@ -580,7 +601,7 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(OCX_RK_W
         }
 #pragma unroll
         for (int m = 0; m < 4; ++m) qc4[m] = qn4[m];
-        if (k + 1 < n) {
+        if (k + 1 < k1) {
             fetch(k + 1);
             fetch_q(k + 1);
         }

@@ -35,3 +35,25 @@ def test_rows_chosen_by_the_size_give_the_bits_of_fixed_rows(gpu, nx, ny, nz, nt
         batch.set_tuning(0, 0)
     assert torch.equal(got, want)
     assert torch.equal(alone.state(0), want)
+
+
+# the layer-marching kernel's columns in one piece, in pieces of 1 .. 5 layers and with a shorter last piece, against
+# the oracle's unsplit columns: every z face of a piece's first and last layer
+@pytest.mark.parametrize("nx,ny,nz,nt", [(20, 18, 1, 1), (40, 33, 7, 2), (130, 70, 11, 1), (300, 250, 13, 3),
+                                         (70, 66, 23, 1)])
+@pytest.mark.parametrize("scheme", ["weno", "js", "up3", "pc"])
+def test_columns_cut_into_pieces_match_the_oracle(gpu, nx, ny, nz, nt, scheme):
+    from oracle import numpy_ref as R
+    print("[gpu case] column pieces", nx, ny, nz, nt, scheme, flush=True)
+    case = synth.regional(nx=nx, ny=ny, nz=nz, nt=nt, seed=7, sigma=True)
+    Fz = torch.from_numpy(np.ascontiguousarray(case.Fz)).cuda()
+    C, V0, V1, Qx, Qy, ok = _dev(case)
+    args = (case.C, case.V0, case.V1, case.Qx, case.Qy, case.Fz, case.ok, case.dt)
+    if scheme == "pc":
+        got = ops.advect_pc(C, V0, V1, Qx, Qy, Fz, ok, case.dt, flags=ops.flags_of(up=3), vert=True)
+        want = R.advect_pc(*args, up_order=3)
+    else:
+        up, js = (3, False) if scheme == "up3" else (0, scheme == "js")
+        got = ops.advect_rk3(C, V0, V1, Qx, Qy, Fz, ok, case.dt, flags=ops.flags_of(js=js, up=up), vert=True)
+        want = R.advect_rk3(*args, z_variant=not js, up_order=up)
+    assert np.array_equal(got.cpu().numpy(), want)
