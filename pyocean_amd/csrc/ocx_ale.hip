@@ -64,7 +64,8 @@ template <int AX>
 void launch_edges(const double* h, const uint8_t* act, double h_min, int n, int ny, int nx, double* lo, double* hi,
                   hipStream_t s) {
     Geo<AX> g{n, ny, nx};
-    k_ppm_edges<AX><<<blocks_for((long long)ny * nx), BS, 0, s>>>(h, act, h_min, g, lo, hi);
+    const dim3 grid(blocks_for((long long)ny * nx), (unsigned)std::min((n + EDGE_LAYERS - 1) / EDGE_LAYERS, 65535));
+    k_ppm_edges<AX><<<grid, BS, 0, s>>>(h, act, h_min, g, lo, hi);
 }
 
 template <int AX>
@@ -91,27 +92,25 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     p.dsum = w.dsum;
     p.notconv = w.notconv;
     p.out = out;
-    const unsigned gb = blocks_for(face_cols(AX, ny, nx));
+    const unsigned gb = (unsigned)((face_cols(AX, ny, nx) + 63) / 64);
     {
         ProfScope _ps("ppm_edges", s);
         launch_edges<AX>(h, act, H_PPM_MIN, n, ny, nx, w.e_lo, w.e_hi, s);
     }
     OCX_TRY(launch_check("ppm edges"));
-    k_fill_u32<<<blocks_for(std::max(max_iter, 1)), BS, 0, s>>>(w.notconv, std::max(max_iter, 1), 0u);
-    OCX_TRY(launch_check("ppm flags"));
     {
         ProfScope _ps("ppm_init", s);
-        k_ppm_init<AX><<<gb, BS, 0, s>>>(p);
+        k_ppm_pass<AX, true><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
     }
     OCX_TRY(launch_check("ppm init"));
     for (int m = 0; m < max_iter; ++m) {
         ProfScope _ps("ppm_newton", s);
-        k_ppm_iter<AX><<<gb, BS, 0, s>>>(p, m);
+        k_ppm_pass<AX, false><<<gb, 64 * PPM_W, 0, s>>>(p, m);
     }
     OCX_TRY(launch_check("ppm newton"));
     {
         ProfScope _ps("ppm_final", s);
-        k_ppm_final<AX><<<gb, BS, 0, s>>>(p);
+        k_ppm_final<AX><<<gb, 64 * PPM_W, 0, s>>>(p);
     }
     return launch_check("ppm final");
 }
@@ -119,8 +118,15 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
 // limiter workspace: r, room (cell stacks), the cut per face column (the larger axis), counters and flags
 struct OutWs {
     double *r, *room, *delta;
-    unsigned long long *count, *bad_face, *key, *idx;
-    unsigned* any;
+    unsigned long long *key, *idx;
+    struct OutFlags* flags;
+};
+
+// the limiter's counters, read by the host in one copy: cell-layers over the bound; per axis the first face whose cut
+// cannot be given back (linear index, else ~0); some cell-layer over; some room0 not finite
+struct OutFlags {
+    unsigned long long count, bad_face[2];
+    unsigned any, wild;
 };
 
 size_t out_layout(void* base, int n, int ny, int nx, OutWs* w) {
@@ -130,20 +136,18 @@ size_t out_layout(void* base, int n, int ny, int nx, OutWs* w) {
     t.r = cv.take<double>(cells);
     t.room = cv.take<double>(cells);
     t.delta = cv.take<double>((size_t)std::max(face_cols(0, ny, nx), face_cols(1, ny, nx)));
-    t.count = cv.take<unsigned long long>(1);
-    t.bad_face = cv.take<unsigned long long>(1);
+    t.flags = cv.take<OutFlags>(1);
     t.key = cv.take<unsigned long long>(1);
     t.idx = cv.take<unsigned long long>(1);
-    t.any = cv.take<unsigned>(1);
     if (w) *w = t;
     return cv.used;
 }
 
-__global__ void k_out_reset(unsigned long long* count, unsigned* any, unsigned long long* bad_face) {
+__global__ void k_out_reset(OutFlags* f, int first) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *count = 0ull;
-        *any = 0u;
-        *bad_face = ~0ull;
+        f->count = 0ull;
+        f->any = f->wild = 0u;
+        if (first) f->bad_face[0] = f->bad_face[1] = ~0ull;
     }
 }
 
@@ -151,24 +155,16 @@ __global__ void k_set_u64(unsigned long long* p, unsigned long long v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
 }
 
-struct OverResult {
-    unsigned long long count;
-    unsigned any;
-    unsigned long long bad_face;
-};
-
 // one over-the-bound test (and r), then the counters to the host (synchronous)
-int over_pass(OutArgs& o, const OutWs& w, double factor, int first, hipStream_t s, OverResult* res) {
-    k_out_reset<<<1, 64, 0, s>>>(w.count, w.any, w.bad_face);
+int over_pass(OutArgs& o, const OutWs& w, double factor, int first, hipStream_t s, OutFlags* res) {
+    k_out_reset<<<1, 64, 0, s>>>(w.flags, first);
     OCX_TRY(launch_check("outflow reset"));
     {
         ProfScope _ps("outflow_over", s);
         k_out_over<<<blocks_for((long long)o.n * o.ny * o.nx), BS, 0, s>>>(o, factor, first);
     }
     OCX_TRY(launch_check("outflow over"));
-    OCX_TRY(hip_check(hipMemcpyAsync(&res->count, w.count, sizeof(unsigned long long), hipMemcpyDeviceToHost, s),
-                      "outflow count"));
-    OCX_TRY(hip_check(hipMemcpyAsync(&res->any, w.any, sizeof(unsigned), hipMemcpyDeviceToHost, s), "outflow flag"));
+    OCX_TRY(hip_check(hipMemcpyAsync(res, w.flags, sizeof *res, hipMemcpyDeviceToHost, s), "outflow counters"));
     return hip_check(hipStreamSynchronize(s), "outflow sync");
 }
 
@@ -214,8 +210,12 @@ int ocx_transport_velocity_f64(const double* u_new, const double* u_old, const u
     for (int q = 0; q < 8; ++q) OCX_TRY(need(p[q], nm[q]));
     hipStream_t s = static_cast<hipStream_t>(stream);
     ProfScope _ps("transport_velocity", s);
-    k_transport_velocity<<<blocks_for(columns), BS, 0, s>>>(u_new, u_old, last_wet, w, L, D, theta, theta_bc, n,
-                                                            columns, ut, Q_bt);
+    if (n <= TV_MAX)
+        k_transport_velocity<<<(unsigned)((columns + 63) / 64), 64 * TV_W, (size_t)n * 2 * 64 * sizeof(double), s>>>(
+            u_new, u_old, last_wet, w, L, D, theta, theta_bc, n, columns, ut, Q_bt);
+    else
+        k_transport_velocity_deep<<<blocks_for(columns), BS, 0, s>>>(u_new, u_old, last_wet, w, L, D, theta, theta_bc,
+                                                                     n, columns, ut, Q_bt);
     return launch_check("transport_velocity");
 }
 
@@ -357,12 +357,12 @@ int ocx_limit_outflow_f64(const double* h, double* Qx, double* Qy, const double*
     o.r = w.r;
     o.room = w.room;
     o.delta = w.delta;
-    o.count = w.count;
-    o.any = w.any;
-    o.bad_face = w.bad_face;
+    o.count = &w.flags->count;
+    o.any = &w.flags->any;
+    o.wild = &w.flags->wild;
     *n_limited = 0;
     if (where) where[0] = where[1] = where[2] = -1;
-    OverResult res{};
+    OutFlags res{};
     OCX_TRY(over_pass(o, w, 1.0, 1, s, &res));
     if (!res.any) {
         *status = OCX_OUTFLOW_NOOP;
@@ -376,11 +376,15 @@ int ocx_limit_outflow_f64(const double* h, double* Qx, double* Qy, const double*
     long long nl = 0;
     for (int pass = 0; pass < max_pass; ++pass) {
         nl += (long long)res.count;
+        // both axes, then the test, then one wait for all counters; the first axis' bad face comes first, as it would
+        // if the host had looked between the two
+        o.bad_face = &w.flags->bad_face[0];
+        OCX_TRY(cut_and_give<0>(o, periodic_x != 0, s));
+        o.bad_face = &w.flags->bad_face[1];
+        OCX_TRY(cut_and_give<1>(o, periodic_y != 0, s));
+        OCX_TRY(over_pass(o, w, factor, 0, s, &res));
         for (int ax = 0; ax < 2; ++ax) {
-            OCX_TRY(ax == 0 ? cut_and_give<0>(o, periodic_x != 0, s) : cut_and_give<1>(o, periodic_y != 0, s));
-            unsigned long long bad = 0;
-            OCX_TRY(hip_check(hipMemcpyAsync(&bad, w.bad_face, sizeof bad, hipMemcpyDeviceToHost, s), "outflow bad"));
-            OCX_TRY(hip_check(hipStreamSynchronize(s), "outflow sync"));
+            const unsigned long long bad = res.bad_face[ax];
             if (bad != ~0ull) {
                 *n_limited = nl;
                 *status = OCX_OUTFLOW_EMPTY_DONOR;
@@ -395,7 +399,6 @@ int ocx_limit_outflow_f64(const double* h, double* Qx, double* Qy, const double*
                             (long long)bad % nf);
             }
         }
-        OCX_TRY(over_pass(o, w, factor, 0, s, &res));
         if (!res.any) {
             *n_limited = nl;
             *status = OCX_OUTFLOW_OK;

@@ -78,12 +78,10 @@ struct Geo {
     }
 };
 
-__device__ __forceinline__ long long gtid() { return (long long)blockIdx.x * blockDim.x + threadIdx.x; }
+// layers whose loads a column's thread issues together
+constexpr int KB = 8;
 
-__global__ void k_fill_u32(unsigned* p, int n, unsigned v) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
+__device__ __forceinline__ long long gtid() { return (long long)blockIdx.x * blockDim.x + threadIdx.x; }
 
 // one lane per wave with `bad` set ORs 1 into *flag (a vector atomic)
 __device__ __forceinline__ void wave_flag(bool bad, unsigned* flag) {
@@ -92,12 +90,78 @@ __device__ __forceinline__ void wave_flag(bool bad, unsigned* flag) {
 }
 
 // ------------------------------------------------------------------------------------------ transport velocity
-// u (n, M) columns; last_wet (M) bytes; w (n, M); L, D (M).  ut (n, M), Qb (M).
-__global__ void k_transport_velocity(const double* __restrict__ u_new, const double* __restrict__ u_old,
-                                     const uint8_t* __restrict__ last_wet, const double* __restrict__ w,
-                                     const double* __restrict__ L, const double* __restrict__ D, double theta,
-                                     double theta_bc, int n, long long M, double* __restrict__ ut,
-                                     double* __restrict__ Qb) {
+// u (n, M) columns; last_wet (M) bytes; w (n, M); L, D (M).  ut (n, M), Qb (M).  Columns of up to TV_MAX layers.
+//
+// A workgroup holds 64 columns; its TV_W wavefronts share the layers, every one of them TV_L layers in registers, all
+// loads in flight together, so that the column is read once (32 B a cell-layer with the result; a thread that walks
+// its column twice fetched 54) and a small grid does not wait at every layer.  The sums run from the bed up as the
+// reference adds: the products go to LDS as [layer][column] and one wavefront per sum adds them in order.  Layers
+// w, w + TV_W, ... belong to wavefront w.  Dynamic LDS: 2 n * 64 doubles.  198 x 159 x 50 42 -> 17 us a direction,
+// 384 x 384 x 50 79 -> 72.
+constexpr int TV_W = 4, TV_L = 16, TV_MAX = TV_W * TV_L;
+__global__ __launch_bounds__(64 * TV_W) void k_transport_velocity(
+    const double* __restrict__ u_new, const double* __restrict__ u_old, const uint8_t* __restrict__ last_wet,
+    const double* __restrict__ w, const double* __restrict__ L, const double* __restrict__ D, double theta,
+    double theta_bc, int n, long long M, double* __restrict__ ut, double* __restrict__ Qb) {
+    extern __shared__ double tv_lds[];
+    double* s1 = tv_lds;
+    double* s0 = tv_lds + (size_t)n * 64;
+    const int lane = threadIdx.x & 63, wv = wave_id();
+    const long long p0 = (long long)blockIdx.x * 64 + lane, p = p0 < M ? p0 : M - 1;
+    const bool wet = last_wet[p] != 0;
+    double un[TV_L], uo[TV_L], ww[TV_L];
+#pragma unroll
+    for (int q = 0; q < TV_L; ++q) {
+        const int k = wv + q * TV_W;
+        if (k < n) {
+            const size_t x = (size_t)k * M + p;
+            un[q] = u_new[x];
+            ww[q] = w[x];
+            uo[q] = wet ? u_old[x] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < TV_L; ++q) {
+        const int k = wv + q * TV_W;
+        if (k < n) {
+            s1[k * 64 + lane] = ww[q] * un[q];
+            s0[k * 64 + lane] = ww[q] * uo[q];
+        }
+    }
+    __syncthreads();
+    double m = 0.0;
+    if (wv < 2) {
+        const double* t = (wv == 0 ? s1 : s0) + lane;
+        for (int k = 0; k < n; ++k) m += t[k * 64];
+    }
+    __syncthreads();
+    if (wv < 2) tv_lds[wv * 64 + lane] = m;
+    __syncthreads();
+    const double d = (theta - theta_bc) * (tv_lds[lane] - tv_lds[64 + lane]);
+    const double omt = 1.0 - theta_bc;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < TV_L; ++q) {
+        const int k = wv + q * TV_W;
+        if (k < n) {
+            const double v = theta_bc * un[q] + omt * uo[q] + d;
+            if (p0 < M) ut[(size_t)k * M + p] = v;
+            s1[k * 64 + lane] = ww[q] * v;
+        }
+    }
+    __syncthreads();
+    if (wv != 0 || p0 >= M) return;
+    double s = 0.0;
+    for (int k = 0; k < n; ++k) s += s1[k * 64 + lane];
+    Qb[p] = L[p] * D[p] * s;
+}
+
+// The same for deeper columns: one thread per column, two walks over its layers.
+__global__ void k_transport_velocity_deep(const double* __restrict__ u_new, const double* __restrict__ u_old,
+                                          const uint8_t* __restrict__ last_wet, const double* __restrict__ w,
+                                          const double* __restrict__ L, const double* __restrict__ D, double theta,
+                                          double theta_bc, int n, long long M, double* __restrict__ ut,
+                                          double* __restrict__ Qb) {
     const long long p = gtid();
     if (p >= M) return;
     const bool wet = last_wet[p] != 0;
@@ -148,14 +212,24 @@ __global__ void k_face_thickness(const double* __restrict__ h, const double* __r
         He = He == He ? He : 0.0;
         const double z_bed = amax(-Hw, -He);
         double sw = 0.0, se = 0.0;
-        for (int k = 0; k < g.n; ++k) {
-            double hw = h[k * PC + cw], he = h[k * PC + ce];
-            hw = hw == hw ? hw : 0.0;
-            he = he == he ? he : 0.0;
-            sw += hw;
-            se += he;
-            qe[k * PF + fo] = amin(hw, amax(0.0, (-Hw + sw) - z_bed));
-            qw[k * PF + fo] = amin(he, amax(0.0, (-He + se) - z_bed));
+        for (int k = 0; k < g.n; k += KB) {
+            double hw[KB], he[KB];
+#pragma unroll
+            for (int q = 0; q < KB; ++q) {
+                const size_t x = (size_t)min(k + q, g.n - 1) * PC;
+                hw[q] = h[x + cw];
+                he[q] = h[x + ce];
+            }
+#pragma unroll
+            for (int q = 0; q < KB; ++q) {
+                if (k + q < g.n) {
+                    const double a0 = hw[q] == hw[q] ? hw[q] : 0.0, a1 = he[q] == he[q] ? he[q] : 0.0;
+                    sw += a0;
+                    se += a1;
+                    qe[(k + q) * PF + fo] = amin(a0, amax(0.0, (-Hw + sw) - z_bed));
+                    qw[(k + q) * PF + fo] = amin(a1, amax(0.0, (-He + se) - z_bed));
+                }
+            }
         }
     } else {
         for (int k = 0; k < g.n; ++k) {
@@ -178,8 +252,11 @@ __device__ __forceinline__ double ppm_slope(double hm1, double hc, double hp1, d
     return mw * me * m > 0.0 ? s : 0.0;
 }
 
-// one thread per cell (natural index j * nx + i), looping over the layers.  The thickness is read as the flux
+// one thread per cell (natural index j * nx + i) and every gridDim.y-th layer (about EDGE_LAYERS of them), which no
+// result of another layer enters: with all layers in one thread a small grid was one long chain of loads per wavefront
+// (198 x 159 x 50: 78-110 us a direction -> 21).  The thickness is read as the flux
 // passes it: inactive cells 0, NaN 0.  Edges: lo = the low-index (west / south) edge, hi = the high one.
+constexpr int EDGE_LAYERS = 4;
 template <int AX>
 __global__ void k_ppm_edges(const double* __restrict__ h, const uint8_t* __restrict__ act, double h_min, Geo<AX> g,
                             double* __restrict__ e_lo, double* __restrict__ e_hi) {
@@ -201,7 +278,7 @@ __global__ void k_ppm_edges(const double* __restrict__ h, const uint8_t* __restr
         m[d] = ex[d] && act[o[d]] ? 1.0 : 0.0;
     }
     const double r6 = 1.0 / 6.0;
-    for (int k = 0; k < g.n; ++k) {
+    for (int k = (int)blockIdx.y; k < g.n; k += (int)gridDim.y) {
         double v[5];
         for (int d = 0; d < 5; ++d) v[d] = m[d] != 0.0 ? nan0(h[k * PC + o[d]]) : 0.0;
         // hm1 / hp1 / slope of the cell at offset d (1..3) with its neighbours d-1, d+1
@@ -255,163 +332,249 @@ struct PpmArgs {
 struct Column {
     size_t cw, ce, fo;
     double dxw, dxe, Lf, Qb;
+    Recip rw, re;            // reciprocals of the widths (qdiv_r gives the IEEE quotient)
     bool open;
 };
 
 template <int AX>
-__device__ __forceinline__ Column column(const PpmArgs<AX>& p, int a, int f) {
+__device__ __forceinline__ Column column(const PpmArgs<AX>& p, long long t) {
     Column c;
+    int a, f;
+    p.g.col(t, a, f);
     const int nc = p.g.ncell();
     c.cw = p.g.cell(a, f > 0 ? f - 1 : 0);
     c.ce = p.g.cell(a, f < nc ? f : nc - 1);
     c.fo = p.g.face(a, f);
     c.dxw = p.dxt[c.cw];
     c.dxe = p.dxt[c.ce];
+    c.rw = recip_of(c.dxw);
+    c.re = recip_of(c.dxe);
     c.Lf = p.L[c.fo];
     c.Qb = p.Qb[c.fo];
     c.open = p.act[c.cw] && p.act[c.ce];
     return c;
 }
 
-// (F, dF/du) of layer k at velocity u: the swept mean thickness of the donor parabola over the Courant fraction,
-// capped by the transport thickness where that is below the donor layer
+// The sums over the layers of a face column run from the bed up, in one chain of additions as the reference adds;
+// everything before the additions is independent from layer to layer.  So a workgroup holds 64 face columns and its
+// PPM_W wavefronts share the layers of a chunk, PPM_L each, with the loads of those layers in flight together; the
+// terms go to LDS as [layer][column], and one wavefront per sum adds them in order while the others load the next
+// chunk (two buffers, one barrier a chunk).  With one thread for a whole column a small grid had fewer wavefronts than
+// SIMDs and waited twice per layer (198 x 159 x 50: a Newton pass 53 us -> 13, the fluxes 90 -> 26; 384 x 384 x 50: 90 -> 54
+// and 155 -> 106; 1024 x 1024 x 50, where both stream, the whole transport 14.3 -> 12.4 ms).
+constexpr int PPM_W = 4, PPM_L = 4, PPM_C = PPM_W * PPM_L;
+
+// terms of the layers k .. k + PPM_L - 1 (beyond n: repeated, not added): F and dF/du at velocity u^theta + du: the
+// swept mean thickness of the donor parabola over the Courant fraction, capped by the transport thickness where that
+// is below the donor layer.  u: the velocities u^theta of these layers.
 template <int AX>
-__device__ __forceinline__ void face_flux(const PpmArgs<AX>& p, const Column& c, int k, double u, double& F,
-                                          double& dF) {
+__device__ __forceinline__ void layer_fluxes(const PpmArgs<AX>& p, const Column& c, int k, const double* u, double* F,
+                                             double* dF) {
     const size_t PC = p.g.pc(), PF = p.g.pf();
-    const bool pos = u >= 0.0;
-    const size_t ci = k * PC + (pos ? c.cw : c.ce);
-    const double cr = amin(fabs(u) * p.dt / (pos ? c.dxw : c.dxe), 1.0);
-    const double hu = nan0(p.h[ci]);
-    const double ww = p.e_lo[ci], ee = p.e_hi[ci];
-    const double curv3 = (ww + ee) - 2.0 * hu;
-    const double dh = pos ? ww - ee : ee - ww;
-    const double edge = pos ? ee : ww;
-    const double q = pos ? p.qe[k * PF + c.fo] : p.qw[k * PF + c.fo];
-    double mean = edge + cr * (0.5 * dh + curv3 * (cr - 1.5));
-    double marg = edge + cr * (dh + 3.0 * curv3 * (cr - 1.0));
-    if (q < hu) {
-        mean = amin(mean, q);
-        marg = amin(marg, q);
+    double hu[PPM_L], ww[PPM_L], ee[PPM_L], qq[PPM_L];
+#pragma unroll
+    for (int q = 0; q < PPM_L; ++q) {
+        const size_t kk = (size_t)min(k + q, p.g.n - 1);
+        const bool pos = u[q] >= 0.0;
+        const size_t ci = kk * PC + (pos ? c.cw : c.ce);
+        hu[q] = p.h[ci];
+        ww[q] = p.e_lo[ci];
+        ee[q] = p.e_hi[ci];
+        qq[q] = (pos ? p.qe : p.qw)[kk * PF + c.fo];
     }
-    F = c.Lf * u * amax(mean, 0.0);
-    dF = c.Lf * amax(marg, 0.0);
-}
-
-template <int AX>
-__device__ __forceinline__ void column_sums(const PpmArgs<AX>& p, const Column& c, double du, double& s,
-                                            double& sd) {
-    s = 0.0;
-    sd = 0.0;
-    if (!c.open) return;
-    const size_t PF = p.g.pf();
-    for (int k = 0; k < p.g.n; ++k) {
-        double F, dF;
-        face_flux(p, c, k, p.ut[k * PF + c.fo] + du, F, dF);
-        s += F;
-        sd += dF;
+#pragma unroll
+    for (int q = 0; q < PPM_L; ++q) {
+        const bool pos = u[q] >= 0.0;
+        const double cr = amin(qdiv_r(fabs(u[q]) * p.dt, pos ? c.rw : c.re), 1.0);
+        const double h0 = nan0(hu[q]);
+        const double curv3 = (ww[q] + ee[q]) - 2.0 * h0;
+        const double dh = pos ? ww[q] - ee[q] : ee[q] - ww[q];
+        const double edge = pos ? ee[q] : ww[q];
+        double mean = edge + cr * (0.5 * dh + curv3 * (cr - 1.5));
+        double marg = edge + cr * (dh + 3.0 * curv3 * (cr - 1.0));
+        if (qq[q] < h0) {
+            mean = amin(mean, qq[q]);
+            marg = amin(marg, qq[q]);
+        }
+        F[q] = c.Lf * u[q] * amax(mean, 0.0);
+        dF[q] = c.Lf * amax(marg, 0.0);
     }
 }
 
-// the CFL bracket [lo, hi] of du and the uncorrected column sums (du = 0 adds nothing: the reference evaluates
-// at u^θ itself)
-template <int AX>
-__global__ void k_ppm_init(PpmArgs<AX> p) {
-    const long long t = gtid();
-    if (t >= p.g.cols()) return;
-    int a, f;
-    p.g.col(t, a, f);
-    const Column c = column(p, a, f);
+// adds the terms of layers [0, m) of one LDS chunk, in order
+__device__ __forceinline__ double add_layers(double s, const double* t, int m) {
+    if (m >= PPM_C) {
+#pragma unroll
+        for (int l = 0; l < PPM_C; ++l) s += t[l * 64];
+    } else {
+        for (int l = 0; l < m; ++l) s += t[l * 64];
+    }
+    return s;
+}
+
+// INIT: the CFL bracket [lo, hi] of du and the uncorrected column sums (the reference evaluates at u^theta itself);
+// block 0 also clears the convergence flags of the passes to come (m of them).
+// Otherwise Newton iteration m (0-based) with bracketing bisection; runs only while the previous iteration left some
+// column unconverged (every column iterates until all have converged, as the reference).
+// Block 64 * PPM_W threads for 64 face columns.
+template <int AX, bool INIT>
+__global__ __launch_bounds__(64 * PPM_W) void k_ppm_pass(PpmArgs<AX> p, int m) {
+    if (!INIT && m > 0 && p.notconv[m - 1] == 0u) return;
+    __shared__ double sF[2][PPM_C * 64], sD[2][PPM_C * 64];
+    const int lane = threadIdx.x & 63, wv = wave_id();
+    if (INIT && blockIdx.x == 0)
+        for (int q = threadIdx.x; q < m; q += 64 * PPM_W) p.notconv[q] = 0u;
+    const long long t0 = (long long)blockIdx.x * 64 + lane;
+    const bool in = t0 < p.g.cols();
+    const long long t = in ? t0 : p.g.cols() - 1;
+    const Column c = column(p, t);
     const size_t PF = p.g.pf();
+    const int n = p.g.n;
     const double limw = 0.5 * c.dxw / p.dt, lime = 0.5 * c.dxe / p.dt;
     double mnw = __builtin_inf(), mxe = -__builtin_inf();
-    double s = 0.0, sd = 0.0;
-    for (int k = 0; k < p.g.n; ++k) {
-        const double u = p.ut[k * PF + c.fo];
-        mnw = amin(mnw, limw - u);
-        mxe = amax(mxe, -(lime + u));
-        if (c.open) {
-            double F, dF;
-            face_flux(p, c, k, u, F, dF);
-            s += F;
-            sd += dF;
-        }
-    }
-    p.hi[t] = amax(amin(limw, mnw), 0.0);
-    p.lo[t] = amin(amax(-lime, mxe), 0.0);
-    p.du[t] = 0.0;
-    p.err[t] = s - c.Qb;
-    p.dsum[t] = sd;
-}
-
-// Newton iteration m (0-based) with bracketing bisection; runs only while the previous iteration left some
-// column unconverged (every column iterates until all have converged, as the reference)
-template <int AX>
-__global__ void k_ppm_iter(PpmArgs<AX> p, int m) {
-    if (m > 0 && p.notconv[m - 1] == 0u) return;
-    const long long t = gtid();
-    bool bad = false;
-    if (t < p.g.cols()) {
-        int a, f;
-        p.g.col(t, a, f);
-        const Column c = column(p, a, f);
+    double nw = 0.0, hi = 0.0, lo = 0.0;
+    if (!INIT) {
         const double e = p.err[t], d = p.du[t], ds = p.dsum[t];
-        double hi = p.hi[t], lo = p.lo[t];
+        hi = p.hi[t];
+        lo = p.lo[t];
         if (e > 0.0) hi = d;
         if (e < 0.0) lo = d;
         const double step = ds > 0.0 ? -e / ds : 0.0;
-        double nw = d + step;
+        nw = d + step;
         if (step > 0.0 && nw >= hi) nw = 0.5 * (d + hi);
         if (step < 0.0 && nw <= lo) nw = 0.5 * (d + lo);
-        double s, sd;
-        column_sums(p, c, nw, s, sd);
-        const double er = s - c.Qb;
-        p.du[t] = nw;
-        p.hi[t] = hi;
-        p.lo[t] = lo;
-        p.err[t] = er;
-        p.dsum[t] = sd;
-        bad = fabs(er) > 1e-12 * amax(fabs(c.Qb), 1.0);
     }
-    wave_flag(bad, p.notconv + m);
+    double sum = 0.0;                       // wavefront 0: of F, 1: of dF/du
+    for (int kc = 0, b = 0; kc < n; kc += PPM_C, b ^= 1) {
+        const int k = kc + wv * PPM_L;
+        double u[PPM_L], F[PPM_L], dF[PPM_L];
+        if (INIT || c.open) {
+#pragma unroll
+            for (int q = 0; q < PPM_L; ++q) u[q] = p.ut[(size_t)min(k + q, n - 1) * PF + c.fo];
+        }
+        if (INIT) {
+#pragma unroll
+            for (int q = 0; q < PPM_L; ++q) {          // (a repeated last layer changes no minimum or maximum)
+                mnw = amin(mnw, limw - u[q]);
+                mxe = amax(mxe, -(lime + u[q]));
+            }
+        }
+        if (c.open) {
+            if (!INIT) {
+#pragma unroll
+                for (int q = 0; q < PPM_L; ++q) u[q] = u[q] + nw;
+            }
+            layer_fluxes(p, c, k, u, F, dF);
+#pragma unroll
+            for (int q = 0; q < PPM_L; ++q) {
+                sF[b][(wv * PPM_L + q) * 64 + lane] = F[q];
+                sD[b][(wv * PPM_L + q) * 64 + lane] = dF[q];
+            }
+        }
+        __syncthreads();
+        if (c.open) {
+            if (wv == 0) sum = add_layers(sum, sF[b] + lane, n - kc);
+            if (wv == 1) sum = add_layers(sum, sD[b] + lane, n - kc);
+        }
+    }
+    if (INIT) {
+        // the wavefronts' brackets meet in LDS (the chunk buffers: every sum is done behind the barrier)
+        __syncthreads();
+        sF[0][wv * 64 + lane] = mnw;
+        sD[0][wv * 64 + lane] = mxe;
+        __syncthreads();
+        if (wv == 0) {
+            for (int q = 1; q < PPM_W; ++q) {
+                mnw = amin(mnw, sF[0][q * 64 + lane]);
+                mxe = amax(mxe, sD[0][q * 64 + lane]);
+            }
+            hi = amax(amin(limw, mnw), 0.0);
+            lo = amin(amax(-lime, mxe), 0.0);
+        }
+    }
+    if (wv == 1 && in) p.dsum[t] = sum;
+    if (wv == 0) {
+        const double er = sum - c.Qb;
+        if (in) {
+            p.du[t] = nw;
+            p.hi[t] = hi;
+            p.lo[t] = lo;
+            p.err[t] = er;
+        }
+        if (!INIT) wave_flag(in && fabs(er) > 1e-12 * amax(fabs(c.Qb), 1.0), p.notconv + m);
+    }
 }
 
-// the layer fluxes at u^θ + du plus the residual R = Q_bt - Σ F shared in proportion to the transport thickness
-// on R's side (the other side's where that column is empty); closed faces 0
+// the layer fluxes at u^theta + du plus the residual R = Q_bt - sum F shared in proportion to the transport thickness
+// on R's side (the other side's where that column is empty); closed faces 0.  The layers are shared by the wavefronts
+// as in k_ppm_pass; the sums of F, q_e and q_w are added by one wavefront each.
 template <int AX>
-__global__ void k_ppm_final(PpmArgs<AX> p) {
-    const long long t = gtid();
-    if (t >= p.g.cols()) return;
-    int a, f;
-    p.g.col(t, a, f);
-    const Column c = column(p, a, f);
+__global__ __launch_bounds__(64 * PPM_W) void k_ppm_final(PpmArgs<AX> p) {
+    __shared__ double sT[2][3][PPM_C * 64];
+    const int lane = threadIdx.x & 63, wv = wave_id();
+    const long long t0 = (long long)blockIdx.x * 64 + lane;
+    const bool in = t0 < p.g.cols();
+    const long long t = in ? t0 : p.g.cols() - 1;
+    const Column c = column(p, t);
     const size_t PF = p.g.pf();
-    if (!c.open) {
-        for (int k = 0; k < p.g.n; ++k) p.out[k * PF + c.fo] = 0.0;
-        return;
-    }
+    const int n = p.g.n;
+    const bool run = in && c.open;
     const double du = p.du[t];
-    double s = 0.0, te = 0.0, tw = 0.0;
-    for (int k = 0; k < p.g.n; ++k) {
-        double F, dF;
-        face_flux(p, c, k, p.ut[k * PF + c.fo] + du, F, dF);
-        p.out[k * PF + c.fo] = F;
-        s += F;
-        te += p.qe[k * PF + c.fo];
-        tw += p.qw[k * PF + c.fo];
+    double sum = 0.0;                       // wavefront 0: of F, 1: of q_e, 2: of q_w
+    for (int kc = 0, b = 0; kc < n; kc += PPM_C, b ^= 1) {
+        const int k = kc + wv * PPM_L;
+        if (run) {
+            double u[PPM_L], F[PPM_L], dF[PPM_L], qe[PPM_L], qw[PPM_L];
+#pragma unroll
+            for (int q = 0; q < PPM_L; ++q) {
+                const size_t x = (size_t)min(k + q, n - 1) * PF + c.fo;
+                u[q] = p.ut[x];
+                qe[q] = p.qe[x];
+                qw[q] = p.qw[x];
+            }
+#pragma unroll
+            for (int q = 0; q < PPM_L; ++q) u[q] = u[q] + du;
+            layer_fluxes(p, c, k, u, F, dF);
+#pragma unroll
+            for (int q = 0; q < PPM_L; ++q) {
+                const int l = (wv * PPM_L + q) * 64 + lane;
+                if (k + q < n) p.out[(size_t)(k + q) * PF + c.fo] = F[q];
+                sT[b][0][l] = F[q];
+                sT[b][1][l] = qe[q];
+                sT[b][2][l] = qw[q];
+            }
+        } else if (in) {
+#pragma unroll
+            for (int q = 0; q < PPM_L; ++q)
+                if (k + q < n) p.out[(size_t)(k + q) * PF + c.fo] = 0.0;
+        }
+        __syncthreads();
+        if (run && wv < 3) sum = add_layers(sum, sT[b][wv] + lane, n - kc);
     }
-    const double R = c.Qb - s;
+    __syncthreads();                        // every sum is done: the buffer takes the three results
+    if (wv < 3) sT[0][wv][lane] = sum;
+    __syncthreads();
+    if (!run) return;
+    const double R = c.Qb - sT[0][0][lane], te = sT[0][1][lane], tw = sT[0][2][lane];
     bool use_e = R >= 0.0;
     double tot = use_e ? te : tw;
     if (tot <= 0.0) {
         use_e = !use_e;
         tot = use_e ? te : tw;
     }
-    const double den = tot > 0.0 ? tot : 1.0;
+    const Recip den = recip_of(tot > 0.0 ? tot : 1.0);
     const double* q = use_e ? p.qe : p.qw;
-    for (int k = 0; k < p.g.n; ++k) {
-        const size_t x = k * PF + c.fo;
-        p.out[x] = p.out[x] + R * q[x] / den;
+    for (int kc = wv * PPM_L; kc < n; kc += PPM_C) {
+        double f[PPM_L], qk[PPM_L];
+#pragma unroll
+        for (int l = 0; l < PPM_L; ++l) {
+            const size_t x = (size_t)min(kc + l, n - 1) * PF + c.fo;
+            f[l] = kc + l < n ? p.out[x] : 0.0;
+            qk[l] = q[x];
+        }
+#pragma unroll
+        for (int l = 0; l < PPM_L; ++l)
+            if (kc + l < n) p.out[(size_t)(kc + l) * PF + c.fo] = f[l] + qdiv_r(R * qk[l], den);
     }
 }
 
@@ -618,6 +781,7 @@ struct OutArgs {
     double* delta;                       // per face column of the current axis
     unsigned long long* count;           // cell-layers over the bound
     unsigned* any;                       // some cell-layer over the bound
+    unsigned* wild;                      // some cell-layer's room0 is not finite
     unsigned long long* bad_face;        // first face whose cut cannot be given back (linear index), else ~0
 };
 
@@ -638,7 +802,7 @@ __device__ __forceinline__ double outflow(const OutArgs& o, int k, int j, int i)
 __global__ void k_out_over(OutArgs o, double factor, int first) {
     const long long t = gtid();
     const size_t PC = (size_t)o.ny * o.nx;
-    bool over = false;
+    bool over = false, wild = false;
     if (t < (long long)(PC * o.n)) {
         const int k = (int)(t / PC);
         const size_t c = (size_t)t - (size_t)k * PC;
@@ -647,7 +811,9 @@ __global__ void k_out_over(OutArgs o, double factor, int first) {
         const double r0 = room0(o, t, c);
         over = o.act[c] && (first ? O > r0 : O > r0 * factor);
         o.r[t] = over ? r0 / (O > 0.0 ? O : 1.0) : 1.0;
+        wild = !(fabs(r0) <= DBL_MAX);
     }
+    wave_flag(wild, o.wild);
     const unsigned long long b = __ballot(over);
     if (b && (threadIdx.x & 63) == (unsigned)(__ffsll((long long)b) - 1)) {
         atomicAdd(o.count, (unsigned long long)__popcll(b));
@@ -700,14 +866,23 @@ __global__ void k_out_cut(OutArgs o, int wrap) {
     double* Q = AX == 0 ? o.Qx : o.Qy;
     const size_t PC = g.pc();
     double d = 0.0;
-    for (int k = 0; k < o.n; ++k) {
-        const size_t x = k * fc.PF + fc.fo;
-        const double q = Q[x];
-        const double rlo = fc.has_lo ? o.r[k * PC + fc.clo] : 1.0;
-        const double rhi = fc.has_hi ? o.r[k * PC + fc.chi] : 1.0;
-        const double nw = q > 0.0 ? q * rlo : (q < 0.0 ? q * rhi : q);
-        d += q - nw;
-        Q[x] = nw;
+    for (int k = 0; k < o.n; k += KB) {
+        double q[KB], rlo[KB], rhi[KB];
+#pragma unroll
+        for (int l = 0; l < KB; ++l) {
+            const size_t kk = (size_t)min(k + l, o.n - 1);
+            q[l] = Q[kk * fc.PF + fc.fo];
+            rlo[l] = fc.has_lo ? o.r[kk * PC + fc.clo] : 1.0;
+            rhi[l] = fc.has_hi ? o.r[kk * PC + fc.chi] : 1.0;
+        }
+#pragma unroll
+        for (int l = 0; l < KB; ++l) {
+            if (k + l < o.n) {
+                const double nw = q[l] > 0.0 ? q[l] * rlo[l] : (q[l] < 0.0 ? q[l] * rhi[l] : q[l]);
+                d += q[l] - nw;
+                if (nw != q[l]) Q[(size_t)(k + l) * fc.PF + fc.fo] = nw;
+            }
+        }
     }
     o.delta[t] = d;
 }
@@ -725,29 +900,61 @@ __global__ void k_out_give(OutArgs o, int wrap) {
     const size_t PC = g.pc();
     const double delta = o.delta[t];
     const double s = sgn(delta);
-    auto room_of = [&](int k, bool lo_side) -> double {
-        const bool has = lo_side ? fc.has_lo : fc.has_hi;
-        return amax(has ? o.room[k * PC + (lo_side ? fc.clo : fc.chi)] : 0.0, 0.0);
-    };
-    auto rm_of = [&](int k, double q) -> double {
-        const bool same = (sgn(q) == s) && (q != 0.0) && (s != 0.0);
-        return same ? (s > 0.0 ? room_of(k, true) : room_of(k, false)) : 0.0;
+    // Most faces have no cut.  There (and where no room0 is infinite or NaN, whose product with 0 would be NaN) the
+    // steps below add +0 to each flux and nothing else: a zero loses its sign.
+    const bool plain = *o.wild == 0u;
+    if (delta == 0.0 && plain) {
+        for (int k = 0; k < o.n; k += KB) {
+            double q[KB];
+#pragma unroll
+            for (int l = 0; l < KB; ++l) q[l] = Q[(size_t)min(k + l, o.n - 1) * fc.PF + fc.fo];
+#pragma unroll
+            for (int l = 0; l < KB; ++l)
+                if (k + l < o.n && q[l] == 0.0 && __double_as_longlong(q[l]) < 0)
+                    Q[(size_t)(k + l) * fc.PF + fc.fo] = 0.0;
+        }
+        return;
+    }
+    // the donor of the cut's direction: the low side for s > 0, else the high side
+    const bool lo_side = s > 0.0, has = lo_side ? fc.has_lo : fc.has_hi;
+    const size_t dc = lo_side ? fc.clo : fc.chi;
+    double q[KB], rm[KB];
+    // fluxes and donor rooms of the layers k .. k + KB - 1 (rm: 0 where a layer takes nothing back)
+    auto load = [&](int k) {
+#pragma unroll
+        for (int l = 0; l < KB; ++l) {
+            const size_t kk = (size_t)min(k + l, o.n - 1);
+            q[l] = Q[kk * fc.PF + fc.fo];
+            rm[l] = has ? o.room[kk * PC + dc] : 0.0;
+        }
+#pragma unroll
+        for (int l = 0; l < KB; ++l) rm[l] = (sgn(q[l]) == s) && (q[l] != 0.0) && (s != 0.0) ? amax(rm[l], 0.0) : 0.0;
     };
     double tot = 0.0;
-    for (int k = 0; k < o.n; ++k) tot += rm_of(k, Q[k * fc.PF + fc.fo]);
+    for (int k = 0; k < o.n; k += KB) {
+        load(k);
+#pragma unroll
+        for (int l = 0; l < KB; ++l)
+            if (k + l < o.n) tot += rm[l];
+    }
     const double need_ = fabs(delta);
     const double give = npmin(need_, tot);
     const double gq = tot > 0.0 ? give / tot : 0.0;
     double cap = 0.0;
-    for (int k = 0; k < o.n; ++k) {
-        const size_t x = k * fc.PF + fc.fo;
-        const double q = Q[x];
-        const double nq = q + s * rm_of(k, q) * gq;
-        Q[x] = nq;
-        const bool opp = (sgn(nq) == -s) && (s != 0.0);
-        cap += opp ? fabs(nq) : 0.0;
+    for (int k = 0; k < o.n; k += KB) {
+        load(k);
+#pragma unroll
+        for (int l = 0; l < KB; ++l) {
+            if (k + l < o.n) {
+                const double nq = q[l] + s * rm[l] * gq;
+                Q[(size_t)(k + l) * fc.PF + fc.fo] = nq;
+                const bool opp = (sgn(nq) == -s) && (s != 0.0);
+                cap += opp ? fabs(nq) : 0.0;
+            }
+        }
     }
     double rest = need_ - give;
+    if (rest == 0.0 && plain) return;       // what follows would take and add zeros of the fluxes' own signs
     const double take = npmin(rest, cap);
     const double frac = cap > 0.0 ? take / cap : 0.0;
     rest = rest - take;
@@ -755,21 +962,17 @@ __global__ void k_out_give(OutArgs o, int wrap) {
     double tot2 = 0.0;
     for (int k = 0; k < o.n; ++k) {
         const size_t x = k * fc.PF + fc.fo;
-        const double q = Q[x];
-        const bool opp = (sgn(q) == -s) && (s != 0.0);
-        Q[x] = q - (opp ? q * frac : 0.0);
-        const bool lo_side = s > 0.0;
-        const bool has = lo_side ? fc.has_lo : fc.has_hi;
-        const double full = has ? room0(o, k * PC + (lo_side ? fc.clo : fc.chi), lo_side ? fc.clo : fc.chi) : 0.0;
+        const double qk = Q[x];
+        const bool opp = (sgn(qk) == -s) && (s != 0.0);
+        Q[x] = qk - (opp ? qk * frac : 0.0);
+        const double full = has ? room0(o, k * PC + dc, dc) : 0.0;
         tot2 += full * on;
     }
     if (rest > 0.0 && tot2 <= 0.0) atomicMin(o.bad_face, (unsigned long long)t);
     const double gr = tot2 > 0.0 ? rest / tot2 : 0.0;
     for (int k = 0; k < o.n; ++k) {
         const size_t x = k * fc.PF + fc.fo;
-        const bool lo_side = s > 0.0;
-        const bool has = lo_side ? fc.has_lo : fc.has_hi;
-        const double full = has ? room0(o, k * PC + (lo_side ? fc.clo : fc.chi), lo_side ? fc.clo : fc.chi) : 0.0;
+        const double full = has ? room0(o, k * PC + dc, dc) : 0.0;
         Q[x] = Q[x] + s * (full * on) * gr;
     }
 }

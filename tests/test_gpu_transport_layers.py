@@ -1,0 +1,81 @@
+"""
+GPU tests of the layer-transport kernels whose layers are shared by a workgroup's wavefronts, at layer and column
+counts around the edges of their chunks, and of the outflow limiter's short ways, against the oracle's bits.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import numpy_ref as R
+from pyocean_amd import ale, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _d(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _bits(got, want, name):
+    g = got.cpu().numpy()
+    assert np.array_equal(g.view(np.int64), np.ascontiguousarray(want).view(np.int64)), name
+
+
+# chunks of 16 layers (4 a wavefront), 64 layers a column at most in registers, 64 columns a workgroup
+@pytest.mark.parametrize("nx,ny,nz", [(12, 5, 1), (63, 9, 3), (64, 4, 4), (65, 3, 15), (31, 7, 16), (20, 33, 17),
+                                      (16, 16, 63), (17, 11, 64), (9, 14, 65)])
+def test_transports_at_chunk_edges_match_the_oracle(gpu, nx, ny, nz):
+    print("[gpu case] transport chunks", nx, ny, nz, flush=True)
+    a = synth.ale_inputs(nx, ny, nz, seed=3)
+    act = np.asarray(a.active, bool)
+    for u1, u0, wet, w, L, D, dx, ax in ((a.u_new, a.u_old, a.wet_u, a.wu, a.Lu, a.Du, a.dx_t, 0),
+                                         (a.v_new, a.v_old, a.wet_v, a.wv, a.Lv, a.Dv, a.dy_t, 1)):
+        ut, Qb = ale.transport_velocity(_d(u1), _d(u0), _d(wet), _d(w), _d(L), _d(D), a.theta, a.theta_bc)
+        rut, rQb = R.transport_velocity(u1, u0, wet, w, L, D, a.theta, a.theta_bc)
+        _bits(ut, rut, "ut")
+        _bits(Qb, rQb, "Q_bt")
+        qp, qn = ale.face_thickness_axis(_d(a.h), _d(a.H), _d(act), True, ax)
+        got, it = ale.ppm_transport(_d(a.h), ut, _d(L), Qb, qp, qn, _d(act), a.dt, _d(dx), ax, return_iterations=True)
+        sw = (lambda x: x) if ax == 0 else (lambda x: np.ascontiguousarray(np.swapaxes(x, -1, -2)))
+        want, rit = R.ppm_transport_x(sw(a.h), sw(rut), sw(L), sw(rQb), sw(qp.cpu().numpy()), sw(qn.cpu().numpy()),
+                                      sw(act), a.dt, sw(dx), return_iterations=True)
+        assert it == rit
+        _bits(got, sw(want), f"Q axis {ax}")
+
+
+# faces with no cut (a zero flux may lose its sign there), with a cut that all comes back, and a room0 that is not
+# finite (no short way: its product with 0 is a NaN in every layer of the column)
+@pytest.mark.parametrize("wild", [None, np.inf])
+@pytest.mark.parametrize("n", [1, 8, 9, 17])
+def test_limit_outflow_short_ways_match_the_oracle(gpu, n, wild):
+    print("[gpu case] limiter short ways", n, wild, flush=True)
+    rng = np.random.default_rng(n)
+    ny, nx, dt = 9, 13, 100.0
+    h = rng.uniform(1.0, 2.0, (n, ny, nx))
+    area = np.full((ny, nx), 1e4)
+    Qx, Qy = rng.normal(0, 5.0, (n, ny, nx + 1)), rng.normal(0, 5.0, (n, ny + 1, nx))
+    Qx[:, :, [0, -1]], Qy[:, [0, -1]] = 0.0, 0.0
+    Qx[:, 2], Qx[:, 3, ::2] = -0.0, -0.0
+    act = np.ones((ny, nx), bool)
+    h[0, 4, 5] = 1e-3
+    Qx[0, 4, 6] = 40.0
+    if wild is not None:
+        h[n - 1, 7, 9] = wild
+    args = (_d(h), _d(Qx), _d(Qy), _d(area), dt, _d(act))
+    try:
+        with np.errstate(all="ignore"):
+            rx, ry, nl, status = R.limit_outflow(h, Qx, Qy, area, dt, act)
+    except RuntimeError:                       # a column that cannot supply its cut (one layer): refused on both sides
+        with pytest.raises(RuntimeError):
+            ale.limit_outflow(*args)
+        return
+    except IndexError:                         # the oracle's search for the emptied layer finds none among NaNs: no answer
+        return
+    gx, gy, gl = ale.limit_outflow(*args)
+    assert gl == nl and status != "noop"
+    for g, r in ((gx, rx), (gy, ry)):
+        g = g.cpu().numpy()
+        assert np.array_equal(np.isnan(g), np.isnan(r))
+        assert np.array_equal(np.where(np.isnan(g), 0.0, g).view(np.int64), np.where(np.isnan(r), 0.0, r).view(np.int64))
