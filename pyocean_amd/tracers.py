@@ -26,6 +26,7 @@ from . import ops
 from ._native import OPEN_E, OPEN_N, OPEN_S, OPEN_W
 from .contract import Issue, Role
 from .periodic import NONE, TRACER_HALO
+from .staging import Staging
 
 _EDGE_BITS = {"west": OPEN_W, "east": OPEN_E, "south": OPEN_S, "north": OPEN_N}
 SCHEMES = ("weno5", "weno5js", "upwind3", "upwind1")
@@ -68,6 +69,7 @@ class TracerAdvection:
         self.record_open_flux = False
         self.last_open_flux: np.ndarray | None = None
         self._ws = ops.Workspace()
+        self._staging = Staging()
 
     # ------------------------------------------------------------------ contract (tracers.py:104-108)
     def check(self, ctx) -> list[Issue]:
@@ -91,6 +93,13 @@ class TracerAdvection:
         if rk and not sch.startswith("weno5"):
             return ops.flags_of(m, up=1 if sch == "upwind1" else 3)
         return ops.flags_of(m, js=sch != "weno5", unlimited=unlimited)
+
+    def _up(self, a, dtype=np.float64):
+        """``a`` on the GPU, through this component's page-locked buffers."""
+        a = np.asarray(a)
+        a = np.ascontiguousarray(a).view(np.uint8) if (a.dtype, dtype) == (np.bool_, np.uint8) else \
+            np.ascontiguousarray(a, dtype=dtype)
+        return self._staging.up(a, ops.require_gpu())
 
     def _pad(self, t, kind):
         per = self.per
@@ -128,9 +137,9 @@ class TracerAdvection:
             return _empty_result(C, flux_face_i)
         flags = self._flags(unlimited)
         okc = np.broadcast_to(ok, C.shape[1:])
-        d = {k: _dev(v) for k, v in (("C", C), ("V0", V0), ("V1", V1), ("Qx", Qx), ("Qy", Qy))}
-        d["ok"] = _dev(okc, np.uint8)
-        d["inflow"] = None if inflow is None else _dev(inflow)
+        d = {k: self._up(v) for k, v in (("C", C), ("V0", V0), ("V1", V1), ("Qx", Qx), ("Qy", Qy))}
+        d["ok"] = self._up(okc, np.uint8)
+        d["inflow"] = None if inflow is None else self._up(inflow)
         fi = flux_face_i
         if self.per:
             H = TRACER_HALO
@@ -145,10 +154,10 @@ class TracerAdvection:
             if fxi is not None and self.per.y:
                 fxi = fxi[..., TRACER_HALO:fxi.shape[-1] - TRACER_HALO].contiguous()
         if want_open:
-            self.last_open_flux = _host(of)
+            self.last_open_flux = self._staging.down(of)
         if flux_face_i is None:
-            return _host(out)
-        return _host(out), _host(fxi)
+            return self._staging.down(out)
+        return self._staging.down(out), self._staging.down(fxi)
 
     # ------------------------------------------------------------------ the step without limiter (tracers.py:342-375)
     def advect(self, C: np.ndarray, V0: np.ndarray, V1: np.ndarray, Qx: np.ndarray, Qy: np.ndarray,
@@ -169,9 +178,9 @@ class TracerAdvection:
         flags = self._flags(rk=True)
         vert = bool(np.any(np.asarray(Fz) != 0.0))
         okc = np.broadcast_to(ok, C.shape[1:])
-        d = {k: _dev(v) for k, v in (("C", C), ("V0", V0), ("V1", V1), ("Qx", Qx), ("Qy", Qy), ("Fz", Fz))}
-        d["ok"] = _dev(okc, np.uint8)
-        d["inflow"] = None if inflow is None else _dev(inflow)
+        d = {k: self._up(v) for k, v in (("C", C), ("V0", V0), ("V1", V1), ("Qx", Qx), ("Qy", Qy), ("Fz", Fz))}
+        d["ok"] = self._up(okc, np.uint8)
+        d["inflow"] = None if inflow is None else self._up(inflow)
         fi = flux_face_i
         if self.per:
             H = TRACER_HALO
@@ -186,8 +195,8 @@ class TracerAdvection:
             if fxi is not None and self.per.y:
                 fxi = fxi[..., TRACER_HALO:fxi.shape[-1] - TRACER_HALO].contiguous()
         if flux_face_i is None:
-            return _host(out)
-        return _host(out), _host(fxi)
+            return self._staging.down(out)
+        return self._staging.down(out), self._staging.down(fxi)
 
     # ------------------------------------------------------------------ single-stage helpers (tracers.py:153-206)
     def faces_h(self, c: np.ndarray, Qx: np.ndarray, Qy: np.ndarray, ok: np.ndarray, ext: np.ndarray | None = None,
