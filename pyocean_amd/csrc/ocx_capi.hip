@@ -1089,10 +1089,13 @@ int ocx_diffuse_h_f64(const double* T, const double* Tw, const double* h, const 
     for (int q = 0; q < 10; ++q) OCX_TRY(need(need_p[q], need_n[q]));
     if (out == T || out == Tw) return fail(OCX_E_ARG, "out must not alias T or Tw (neighbours are read)");
     if (nz > 65535) return fail(OCX_E_ARG, "nz = %d layers: at most 65535", nz);
-    const dim3 grid((unsigned)((nx + 63) / 64), (unsigned)((ny + 3) / 4), (unsigned)nz), block(64, 4);
+    const long long blocks = (long long)((nx + 63) / 64) * ((ny + DH_Y - 1) / DH_Y) * nz;
+    if (blocks > 0x7fffffffLL) return fail(OCX_E_ARG, "%lld blocks exceed one launch", blocks);
+    const dim3 block(64, DH_Y);
     hipStream_t s = static_cast<hipStream_t>(stream);
     ProfScope _ps("diffuse_h", s);
-    k_diffuse_h<<<grid, block, 0, s>>>(T, Tw, h, act, cx, cy, okx, oky, V, nt, nz, ny, nx, kh, dt, out);
+    (T == Tw ? k_diffuse_h<true> : k_diffuse_h<false>)<<<(unsigned)blocks, block, 0, s>>>(
+        T, Tw, h, act, cx, cy, okx, oky, V, nt, nz, ny, nx, kh, dt, out);
     return launch_check("diffuse_h");
 }
 

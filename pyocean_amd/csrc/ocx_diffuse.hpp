@@ -19,18 +19,28 @@ namespace ocx {
 
 __device__ __forceinline__ double pymin(double a, double b) { return b < a ? b : a; }   // Python's min(a, b)
 
-// grid (ceil(nx / 64), ceil(ny / 4), n), block (64, 4): one thread per cell of layer k for every tracer of the
-// stack (the per-layer fields are read once and serve all tracers); rows are coalesced across lanes
-__global__ __launch_bounds__(256) void k_diffuse_h(const double* __restrict__ T, const double* __restrict__ Tw,
+// One thread per cell of layer k for every tracer of the stack (the per-layer fields are read once and serve all
+// tracers), block (64, DH_Y); rows are coalesced across lanes.  The blocks are a 1-D grid, x fastest, then y, then k,
+// remapped XCD-contiguously, so that the rows a block shares with those north and south of it come from one L2 (in
+// dispatch order neighbours sat on different XCDs and each fetched them from memory).  Two tracers' loads are in flight
+// together, the volume's reciprocal is refined once for all tracers (qdiv_r gives the IEEE quotient), and a T that is
+// Tw is not read twice.  Bound by memory (20 B a tracer-cell, 3.5 TB/s): 701 x 523 x 50 x 10 1186 us -> 1040,
+// 384 x 384 x 50 x 10 449 -> 408; blocks of 8 or 16 rows 1048 and 1052.
+constexpr int DH_Y = 4;
+template <bool SAME>
+__global__ __launch_bounds__(64 * DH_Y) void k_diffuse_h(const double* __restrict__ T, const double* __restrict__ Tw,
                                                    const double* __restrict__ h, const uint8_t* __restrict__ act,
                                                    const double* __restrict__ cx, const double* __restrict__ cy,
                                                    const uint8_t* __restrict__ okx, const uint8_t* __restrict__ oky,
                                                    const double* __restrict__ V, int nt, int n, int ny, int nx,
                                                    double kh, double dt, double* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
+    const int gx = (nx + 63) / 64, gy = (ny + DH_Y - 1) / DH_Y;
+    long long L = xcd_logical((long long)blockIdx.x, (long long)gridDim.x);
+    const int i = (int)(L % gx) * 64 + threadIdx.x;
+    L /= gx;
+    const int j = (int)(L % gy) * DH_Y + threadIdx.y, k = (int)(L / gy);
     if (i >= nx || j >= ny) return;
     const size_t plane = (size_t)ny * nx;
-    const int k = blockIdx.z;
     const double* hk = h + (size_t)k * plane;
     const double* Vk = V + (size_t)k * plane;
     const size_t c = (size_t)j * nx + i;
@@ -46,20 +56,30 @@ __global__ __launch_bounds__(256) void k_diffuse_h(const double* __restrict__ T,
     const bool fnk = hn && oky[c + nx] != 0;
     const double cxw = cx[fx], cxe = cx[fx + 1], cys = cy[c], cyn = cy[c + nx];
     const double v0 = Vk[c];
-    const double huw = (aw && a0) ? pymin(hw_, h0) : 0.0, hue = (a0 && ae) ? pymin(h0, he_) : 0.0;
-    const double hvs = (as && a0) ? pymin(hs_, h0) : 0.0, hvn = (a0 && an) ? pymin(h0, hn_) : 0.0;
-    for (int t = 0; t < nt; ++t) {
-        const size_t pl = ((size_t)t * n + k) * plane;
+    const Recip rv = recip_of(v0);
+    // -kh L/dx h of the faces, in the reference's order
+    const double gw = -kh * cxw * ((aw && a0) ? pymin(hw_, h0) : 0.0), ge = -kh * cxe * ((a0 && ae) ? pymin(h0, he_) : 0.0);
+    const double gs = -kh * cys * ((as && a0) ? pymin(hs_, h0) : 0.0), gn = -kh * cyn * ((a0 && an) ? pymin(h0, hn_) : 0.0);
+    const size_t step = (size_t)n * plane;
+    auto cell = [&](size_t pl) {
         const double* Wp = Tw + pl;
         const double w0 = Wp[c], ww = Wp[cw], we = Wp[ce], ws = Wp[cs], wn = Wp[cn];
-        const double t0 = T[pl + c];
-        const double fw = fwk ? -kh * cxw * huw * (w0 - ww) : 0.0;
-        const double fe = fek ? -kh * cxe * hue * (we - w0) : 0.0;
-        const double fs = fsk ? -kh * cys * hvs * (w0 - ws) : 0.0;
-        const double fn = fnk ? -kh * cyn * hvn * (wn - w0) : 0.0;
+        const double t0 = SAME ? w0 : T[pl + c];
+        const double fw = fwk ? gw * (w0 - ww) : 0.0;
+        const double fe = fek ? ge * (we - w0) : 0.0;
+        const double fs = fsk ? gs * (w0 - ws) : 0.0;
+        const double fn = fnk ? gn * (wn - w0) : 0.0;
         const double div = fe - fw + fn - fs;
-        out[pl + c] = v0 > 0.0 ? t0 - dt * div / v0 : t0;
+        return v0 > 0.0 ? t0 - qdiv_r(dt * div, rv) : t0;
+    };
+    int t = 0;
+    size_t pl = (size_t)k * plane;
+    for (; t + 1 < nt; t += 2, pl += 2 * step) {
+        const double r0 = cell(pl), r1 = cell(pl + step);
+        out[pl + c] = r0;
+        out[pl + step + c] = r1;
     }
+    if (t < nt) out[pl + c] = cell(pl);
 }
 
 // coefficients of layer k of column col: lower, the diagonal and upper of the tridiagonal row

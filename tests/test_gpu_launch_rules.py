@@ -57,3 +57,24 @@ def test_columns_cut_into_pieces_match_the_oracle(gpu, nx, ny, nz, nt, scheme):
         got = ops.advect_rk3(C, V0, V1, Qx, Qy, Fz, ok, case.dt, flags=ops.flags_of(js=js, up=up), vert=True)
         want = R.advect_rk3(*args, z_variant=not js, up_order=up)
     assert np.array_equal(got.cpu().numpy(), want)
+
+
+# the along-layer diffusion reads T once where it is Tw, and takes two tracers at a time: odd counts, ragged blocks
+@pytest.mark.parametrize("nx,ny,nz,nt", [(1, 1, 1, 1), (63, 5, 2, 2), (64, 4, 3, 3), (65, 9, 2, 1), (130, 17, 5, 5)])
+def test_diffusion_of_one_and_of_two_arrays_match_the_oracle(gpu, nx, ny, nz, nt):
+    from oracle import numpy_ref as R
+    print("[gpu case] diffuse_h", nx, ny, nz, nt, flush=True)
+    rng = np.random.default_rng(nx)
+    T = rng.normal(10.0, 2.0, (nt, nz, ny, nx))
+    act = rng.random((ny, nx)) > 0.2
+    h = rng.uniform(0.5, 3.0, (nz, ny, nx)) * act
+    V = h * 1e6
+    cx, cy = rng.uniform(0.9, 1.1, (ny, nx + 1)), rng.uniform(0.9, 1.1, (ny + 1, nx))
+    okx, oky = rng.random((ny, nx + 1)) > 0.1, rng.random((ny + 1, nx)) > 0.1
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()                                   # noqa: E731
+    m = lambda a: d(a.astype(np.uint8))                                                              # noqa: E731
+    args = (d(h), m(act), d(cx), d(cy), m(okx), m(oky), d(V), 100.0, 600.0)
+    want = R.diffuse_h_ale(T, T, h, act, cx, cy, okx, oky, V, 100.0, 600.0)
+    a, b = d(T), d(T)
+    for got in (ops.diffuse_h(a, a, *args), ops.diffuse_h(a, b, *args)):
+        assert np.array_equal(got.cpu().numpy(), want)
