@@ -37,7 +37,7 @@ long long face_cols(int axis, int ny, int nx) {
 
 // PPM workspace: the two edge stacks, the Newton state per face column, the convergence flags
 struct PpmWs {
-    double *e_lo, *e_hi, *du, *lo, *hi, *err, *dsum;
+    double *e_lo, *e_hi, *du, *lo, *hi, *err, *dsum, *hist;
     unsigned* notconv;
 };
 
@@ -56,6 +56,7 @@ size_t ppm_layout(void* base, int n, int ny, int nx, int axis, int max_iter, Ppm
     t.err = cv.take<double>(cols);
     t.dsum = cv.take<double>(cols);
     t.notconv = cv.take<unsigned>((size_t)std::max(max_iter, 1));
+    t.hist = cv.take<double>(cols * (size_t)std::min(std::max(max_iter - PPM_SINGLE, 0), PPM_BUNDLE));
     if (w) *w = t;
     return cv.used;
 }
@@ -91,6 +92,7 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     p.err = w.err;
     p.dsum = w.dsum;
     p.notconv = w.notconv;
+    p.hist = w.hist;
     p.out = out;
     const unsigned gb = (unsigned)((face_cols(AX, ny, nx) + 63) / 64);
     {
@@ -103,14 +105,18 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
         k_ppm_pass<AX, true><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
     }
     OCX_TRY(launch_check("ppm init"));
-    for (int m = 0; m < max_iter; ++m) {
+    for (int m = 0; m < std::min(max_iter, PPM_SINGLE); ++m) {
         ProfScope _ps("ppm_newton", s);
         k_ppm_pass<AX, false><<<gb, 64 * PPM_W, 0, s>>>(p, m);
+    }
+    for (int m = PPM_SINGLE; m < max_iter; m += PPM_BUNDLE) {
+        ProfScope _ps("ppm_newton_bundle", s);
+        k_ppm_bundle<AX><<<gb, 64 * PPM_W, 0, s>>>(p, m, std::min(PPM_BUNDLE, max_iter - m));
     }
     OCX_TRY(launch_check("ppm newton"));
     {
         ProfScope _ps("ppm_final", s);
-        k_ppm_final<AX><<<gb, 64 * PPM_W, 0, s>>>(p);
+        k_ppm_final<AX><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
     }
     return launch_check("ppm final");
 }

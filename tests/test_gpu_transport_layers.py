@@ -45,6 +45,24 @@ def test_transports_at_chunk_edges_match_the_oracle(gpu, nx, ny, nz):
         _bits(got, sw(want), f"Q axis {ax}")
 
 
+# iterations with a launch of their own, and bundles of them: stops before, at and after the ends of both, with columns
+# that never converge (a flux beyond their bracket), that do after 4, and, a flux just inside its bracket, after 23
+@pytest.mark.parametrize("max_iter", [0, 1, 7, 8, 9, 19, 20, 21, 33])
+@pytest.mark.parametrize("reach", [1.0, 50.0, 1.672235424598329])
+def test_iteration_bundles_stop_where_the_oracle_stops(gpu, max_iter, reach):
+    print("[gpu case] newton bundles", max_iter, reach, flush=True)
+    a = synth.ale_inputs(40, 13, 6, seed=4)
+    act = np.asarray(a.active, bool)
+    ut, Qb = R.transport_velocity(a.u_new, a.u_old, a.wet_u, a.wu, a.Lu, a.Du, a.theta, a.theta_bc)
+    qe, qw = R.face_transport_thickness(a.h, a.H, act, True)
+    Qb = Qb * reach
+    want, rit = R.ppm_transport_x(a.h, ut, a.Lu, Qb, qe, qw, act, a.dt, a.dx_t, max_iter, return_iterations=True)
+    got, it = ale.ppm_transport(_d(a.h), _d(ut), _d(a.Lu), _d(Qb), _d(qe), _d(qw), _d(act), a.dt, _d(a.dx_t), 0, max_iter,
+                                return_iterations=True)
+    assert it == rit
+    _bits(got, want, "Q")
+
+
 # faces with no cut (a zero flux may lose its sign there), with a cut that all comes back, and a room0 that is not
 # finite (no short way: its product with 0 is a NaN in every layer of the column)
 @pytest.mark.parametrize("wild", [None, np.inf])
