@@ -22,7 +22,9 @@ __device__ __forceinline__ double pymin(double a, double b) { return b < a ? b :
 // One thread per cell of layer k for every tracer of the stack (the per-layer fields are read once and serve all
 // tracers), block (64, DH_Y); rows are coalesced across lanes.  The blocks are a 1-D grid, x fastest, then y, then k,
 // remapped XCD-contiguously, so that the rows a block shares with those north and south of it come from one L2 (in
-// dispatch order neighbours sat on different XCDs and each fetched them from memory).  Two tracers' loads are in flight
+// dispatch order neighbours sat on different XCDs and each fetched them from memory).  Where a row has a multiple of 8
+// blocks, dispatch order itself puts a block and its north and south neighbours on one XCD, and the 8 XCDs stay on
+// neighbouring rows: 1024 x 1024 x 50 x 10 3257 us, remapped 3375 (701 x 523 x 50 x 10 1242 and 1200).  Two tracers' loads are in flight
 // together, the volume's reciprocal is refined once for all tracers (qdiv_r gives the IEEE quotient), and a T that is
 // Tw is not read twice.  Bound by memory (20 B a tracer-cell, 3.5 TB/s): 701 x 523 x 50 x 10 1186 us -> 1040,
 // 384 x 384 x 50 x 10 449 -> 408; blocks of 8 or 16 rows 1048 and 1052.
@@ -35,7 +37,7 @@ __global__ __launch_bounds__(64 * DH_Y) void k_diffuse_h(const double* __restric
                                                    const double* __restrict__ V, int nt, int n, int ny, int nx,
                                                    double kh, double dt, double* __restrict__ out) {
     const int gx = (nx + 63) / 64, gy = (ny + DH_Y - 1) / DH_Y;
-    long long L = xcd_logical((long long)blockIdx.x, (long long)gridDim.x);
+    long long L = gx % 8 == 0 ? (long long)blockIdx.x : xcd_logical((long long)blockIdx.x, (long long)gridDim.x);
     const int i = (int)(L % gx) * 64 + threadIdx.x;
     L /= gx;
     const int j = (int)(L % gy) * DH_Y + threadIdx.y, k = (int)(L / gy);

@@ -60,7 +60,8 @@ def test_columns_cut_into_pieces_match_the_oracle(gpu, nx, ny, nz, nt, scheme):
 
 
 # the along-layer diffusion reads T once where it is Tw, and takes two tracers at a time: odd counts, ragged blocks
-@pytest.mark.parametrize("nx,ny,nz,nt", [(1, 1, 1, 1), (63, 5, 2, 2), (64, 4, 3, 3), (65, 9, 2, 1), (130, 17, 5, 5)])
+@pytest.mark.parametrize("nx,ny,nz,nt", [(1, 1, 1, 1), (63, 5, 2, 2), (64, 4, 3, 3), (65, 9, 2, 1), (130, 17, 5, 5),
+                                         (449, 9, 2, 3), (512, 6, 3, 2)])      # rows of a multiple of 8 blocks
 def test_diffusion_of_one_and_of_two_arrays_match_the_oracle(gpu, nx, ny, nz, nt):
     from oracle import numpy_ref as R
     print("[gpu case] diffuse_h", nx, ny, nz, nt, flush=True)
