@@ -24,10 +24,10 @@ __device__ __forceinline__ double pymin(double a, double b) { return b < a ? b :
 // remapped XCD-contiguously, so that the rows a block shares with those north and south of it come from one L2 (in
 // dispatch order neighbours sat on different XCDs and each fetched them from memory).  Where a row has a multiple of 8
 // blocks, dispatch order itself puts a block and its north and south neighbours on one XCD, and the 8 XCDs stay on
-// neighbouring rows: 1024 x 1024 x 50 x 10 3257 us, remapped 3375 (701 x 523 x 50 x 10 1242 and 1200).  Two tracers' loads are in flight
-// together, the volume's reciprocal is refined once for all tracers (qdiv_r gives the IEEE quotient), and a T that is
-// Tw is not read twice.  Bound by memory (20 B a tracer-cell, 3.5 TB/s): 701 x 523 x 50 x 10 1186 us -> 1040,
-// 384 x 384 x 50 x 10 449 -> 408; blocks of 8 or 16 rows 1048 and 1052.
+// neighbouring rows: 1024 x 1024 x 50 x 10 3257 us, remapped 3375 (701 x 523 x 50 x 10 1242 and 1200).  Two tracers'
+// loads are in flight together, the volume's reciprocal is refined once for all tracers (qdiv_r gives the IEEE
+// quotient), and a T that is Tw is not read twice.  Bound by memory (20 B a tracer-cell, 3.5 TB/s): 701 x 523 x 50 x
+// 10 1186 us -> 1040, 384 x 384 x 50 x 10 449 -> 408; blocks of 8 or 16 rows 1048 and 1052.
 constexpr int DH_Y = 4;
 template <bool SAME>
 __global__ __launch_bounds__(64 * DH_Y) void k_diffuse_h(const double* __restrict__ T, const double* __restrict__ Tw,
