@@ -17,6 +17,15 @@ CHUNK = 8 << 20         # bytes of each of the two buffers: long enough for the 
 DIRECT = 64 << 10       # arrays up to this size are copied directly (one copy, no events)
 
 
+class _Readable:
+    """The memory of an array, which may be read-only, as one that NumPy takes for writable (torch warns of any other;
+    here it is only read)."""
+
+    def __init__(self, a: np.ndarray):
+        self._a = a                      # keeps the memory
+        self.__array_interface__ = dict(a.__array_interface__, data=(a.__array_interface__["data"][0], False))
+
+
 class Staging:
     """Two page-locked buffers, allocated on first use and freed with their owner.  Calls take turns on a lock; the
     copies run on the current stream, and a call returns when the host array may be changed (``up``) or read
@@ -44,8 +53,8 @@ class Staging:
             self._event[b] = None
 
     def up(self, a: np.ndarray, device: torch.device) -> torch.Tensor:
-        """A device tensor with the values of the C-contiguous array ``a``."""
-        t = torch.from_numpy(a)
+        """A device tensor with the values of the C-contiguous array ``a`` (read-only or not)."""
+        t = torch.from_numpy(a if a.flags.writeable else np.asarray(_Readable(a)))
         if a.nbytes <= DIRECT:
             return t.to(device)
         out = torch.empty(t.shape, dtype=t.dtype, device=device)

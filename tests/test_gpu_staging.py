@@ -49,3 +49,24 @@ def test_threads_take_turns(gpu):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_a_step_takes_read_only_arrays_without_a_warning(gpu):
+    import warnings
+
+    from pyocean_amd import synth
+    from pyocean_amd.tracers import OpenEdges, TracerAdvection
+    print("[gpu case] read-only arrays", flush=True)
+    case = synth.regional(nx=70, ny=60, nz=5, nt=2, seed=3)
+    adv = TracerAdvection(scheme="weno5", time="ssprk3", dt=case.dt, ob=OpenEdges(()))
+    args = [case.C.copy(), case.V0, case.V1, case.Qx, case.Qy, np.ascontiguousarray(case.ok, bool)]
+    want = adv.advect_fct(*args)
+    args[0].flags.writeable = False
+    torch.set_warn_always(True)
+    try:
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            got = adv.advect_fct(*args)
+    finally:
+        torch.set_warn_always(False)
+    assert np.array_equal(got, want)
