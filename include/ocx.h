@@ -346,8 +346,9 @@ int ocx_apply_freshwater_f64(double* stack, int nt, int n, int ny, int nx, int t
 /* Outflow limiter, in place on Qx and Qy; host-synchronous (the number of passes depends on the data).
  * Replaces limit_outflow / _give_back / _outflow_exceeds (core/vertical/ale.py:299-437).  check_only: only test
  * whether any active cell-layer sends out more than it holds.  status: OCX_OUTFLOW_*; n_limited: cell-layers scaled
- * over all passes.  On OCX_OUTFLOW_EMPTY_DONOR where = (axis, a, f) of the face; on OCX_OUTFLOW_ACCEPTED /
- * NEGATIVE where = (k, j, i) of the lowest h and value = that h. */
+ * over all passes.  On OCX_OUTFLOW_EMPTY_DONOR where = (axis, a, f) of the face, and the fluxes are those at which the
+ * reference raises: for a u-face (axis 0) Qy is as the passes before left it; on OCX_OUTFLOW_ACCEPTED / NEGATIVE
+ * where = (k, j, i) of the lowest h and value = that h. */
 #define OCX_OUTFLOW_NOOP 0          /* nothing exceeded: Qx, Qy untouched */
 #define OCX_OUTFLOW_OK 1            /* limited; no cell-layer exceeds any more */
 #define OCX_OUTFLOW_ACCEPTED 2      /* still exceeding after max_pass but h >= -h_floor (the reference warns) */

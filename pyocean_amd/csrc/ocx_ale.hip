@@ -382,8 +382,8 @@ int ocx_limit_outflow_f64(const double* h, double* Qx, double* Qy, const double*
     long long nl = 0;
     for (int pass = 0; pass < max_pass; ++pass) {
         nl += (long long)res.count;
-        // both axes, then the test, then one wait for all counters; the first axis' bad face comes first, as it would
-        // if the host had looked between the two
+        // both axes, then the test, then one wait for all counters; the first axis' bad face comes first, and leaves
+        // the second axis as it was, as it would if the host had looked between the two
         o.bad_face = &w.flags->bad_face[0];
         OCX_TRY(cut_and_give<0>(o, periodic_x != 0, s));
         o.bad_face = &w.flags->bad_face[1];

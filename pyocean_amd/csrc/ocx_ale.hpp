@@ -860,8 +860,16 @@ struct OutArgs {
     unsigned long long* count;           // cell-layers over the bound
     unsigned* any;                       // some cell-layer over the bound
     unsigned* wild;                      // some cell-layer's room0 is not finite
-    unsigned long long* bad_face;        // first face whose cut cannot be given back (linear index), else ~0
+    unsigned long long* bad_face;        // first face of the current axis whose cut cannot be given back (linear
+                                         // index), else ~0; bad_face[-1]: the u-faces' while the v-faces run
 };
+
+// Both axes of a pass run before the host looks at the flags.  The v-faces leave everything as it is where a u-face
+// could not place its cut: the call then ends with that face, and Qy keeps what the passes before gave it.
+template <int AX>
+__device__ __forceinline__ bool pass_ended(const OutArgs& o) {
+    return AX == 1 && o.bad_face[-1] != ~0ull;
+}
 
 // what a cell-layer can give in Δt, (h - h_floor)+ A / Δt with A = 0 on land
 __device__ __forceinline__ double room0(const OutArgs& o, size_t x, size_t c) {
@@ -939,7 +947,7 @@ template <int AX>
 __global__ void k_out_cut(OutArgs o, int wrap) {
     const long long t = gtid();
     Geo<AX> g{o.n, o.ny, o.nx};
-    if (t >= g.cols()) return;
+    if (t >= g.cols() || pass_ended<AX>(o)) return;
     const OutFace<AX> fc = out_face<AX>(o, t, wrap);
     double* Q = AX == 0 ? o.Qx : o.Qy;
     const size_t PC = g.pc();
@@ -972,7 +980,7 @@ template <int AX>
 __global__ void k_out_give(OutArgs o, int wrap) {
     const long long t = gtid();
     Geo<AX> g{o.n, o.ny, o.nx};
-    if (t >= g.cols()) return;
+    if (t >= g.cols() || pass_ended<AX>(o)) return;
     const OutFace<AX> fc = out_face<AX>(o, t, wrap);
     double* Q = AX == 0 ? o.Qx : o.Qy;
     const size_t PC = g.pc();

@@ -97,3 +97,47 @@ def test_limit_outflow_short_ways_match_the_oracle(gpu, n, wild):
         g = g.cpu().numpy()
         assert np.array_equal(np.isnan(g), np.isnan(r))
         assert np.array_equal(np.where(np.isnan(g), 0.0, g).view(np.int64), np.where(np.isnan(r), 0.0, r).view(np.int64))
+
+
+# a u-face (or a v-face) with nowhere to place its cut ends the call: on a u-face Qy is still the caller's, on either
+# the fluxes of that pass are the oracle's at the point where it raises
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("n", [1, 3, 9])
+def test_limit_outflow_keeps_the_fluxes_of_the_error(gpu, n, axis):
+    import ctypes
+
+    from pyocean_amd import _native, ops
+    print("[gpu case] limiter error", n, axis, flush=True)
+    rng = np.random.default_rng(5)
+    ny, nx, dt = 9, 13, 100.0
+    h = rng.uniform(1.0, 2.0, (n, ny, nx))
+    area = np.full((ny, nx), 1e4)
+    Qx, Qy = rng.normal(0, 5.0, (n, ny, nx + 1)), rng.normal(0, 5.0, (n, ny + 1, nx))
+    Qx[:, :, [0, -1]], Qy[:, [0, -1]] = 0.0, 0.0
+    act = np.ones((ny, nx), bool)
+    h[:, 4, 5] = 0.0                                  # an empty column that a face must carry its cut out of
+    h[0, 6, 8] = 1e-3                                 # a layer whose cut across a v-face changes Qy
+    Qx[:, 4, 5:7] = Qy[:, 4:6, 5] = 0.0
+    if axis == 0:
+        Qx[:, 4, 6] = 7.0
+    else:
+        Qy[:, 5, 5] = 7.0
+    Qy[0, 7, 8] = 40.0
+    with pytest.raises(RuntimeError):
+        R.limit_outflow(h, Qx, Qy, area, dt, act)
+    want = (Qx.copy(), Qy.copy())
+    dh, dx, dy, da, dm = _d(h), _d(Qx), _d(Qy), _d(area), _d(act.astype(np.uint8))
+    L = _native.lib()
+    ws = torch.empty(int(L.ocx_limit_outflow_workspace_bytes(n, ny, nx)), dtype=torch.uint8, device="cuda")
+    nl, st = ctypes.c_longlong(0), ctypes.c_int(0)
+    where, val = (ctypes.c_longlong * 3)(), ctypes.c_double(0.0)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())                                                      # noqa: E731
+    rc = L.ocx_limit_outflow_f64(p(dh), p(dx), p(dy), p(da), p(dm), n, ny, nx, dt, 2e-10, 50, 0, 0, 0, p(ws), ws.numel(),
+                                 ctypes.byref(nl), ctypes.byref(st), where, ctypes.byref(val), ops._stream())
+    assert rc == _native.OCX_E_RANGE and st.value == _native.OUTFLOW_EMPTY_DONOR
+    assert tuple(where)[:1] == (axis,)
+    face = (4, 6) if axis == 0 else None
+    if face:
+        assert tuple(where)[1:] == face
+        _bits(dy, want[1], "Qy")
+    assert not np.array_equal(dx.cpu().numpy() if axis == 0 else dy.cpu().numpy(), want[axis])
