@@ -1090,11 +1090,10 @@ int ocx_diffuse_h_f64(const double* T, const double* Tw, const double* h, const 
     if (out == T || out == Tw) return fail(OCX_E_ARG, "out must not alias T or Tw (neighbours are read)");
     if (nz > 65535) return fail(OCX_E_ARG, "nz = %d layers: at most 65535", nz);
     const long long blocks = (long long)((nx + 63) / 64) * ((ny + DH_Y - 1) / DH_Y) * nz;
-    if (blocks > 0x7fffffffLL) return fail(OCX_E_ARG, "%lld blocks exceed one launch", blocks);
     const dim3 block(64, DH_Y);
     hipStream_t s = static_cast<hipStream_t>(stream);
     ProfScope _ps("diffuse_h", s);
-    (T == Tw ? k_diffuse_h<true> : k_diffuse_h<false>)<<<(unsigned)blocks, block, 0, s>>>(
+    (T == Tw ? k_diffuse_h<true> : k_diffuse_h<false>)<<<wide_grid(blocks), block, 0, s>>>(
         T, Tw, h, act, cx, cy, okx, oky, V, nt, nz, ny, nx, kh, dt, out);
     return launch_check("diffuse_h");
 }

@@ -37,11 +37,12 @@ __global__ __launch_bounds__(64 * DH_Y) void k_diffuse_h(const double* __restric
                                                    const double* __restrict__ V, int nt, int n, int ny, int nx,
                                                    double kh, double dt, double* __restrict__ out) {
     const int gx = (nx + 63) / 64, gy = (ny + DH_Y - 1) / DH_Y;
-    long long L = gx % 8 == 0 ? (long long)blockIdx.x : xcd_logical((long long)blockIdx.x, (long long)gridDim.x);
+    long long L = block_id();
+    if (gx % 8 != 0) L += xcd_logical((long long)blockIdx.x, (long long)gridDim.x) - blockIdx.x;
     const int i = (int)(L % gx) * 64 + threadIdx.x;
     L /= gx;
     const int j = (int)(L % gy) * DH_Y + threadIdx.y, k = (int)(L / gy);
-    if (i >= nx || j >= ny) return;
+    if (i >= nx || j >= ny || k >= n) return;
     const size_t plane = (size_t)ny * nx;
     const double* hk = h + (size_t)k * plane;
     const double* Vk = V + (size_t)k * plane;

@@ -56,6 +56,15 @@ struct Carver {
     }
 };
 
+// The grid of a 1-D launch of any length: a launch counts the threads of each dimension in 32 bits, so blocks beyond
+// 2^22 (of at most 512 threads) go to the second dimension.  The kernel takes its block from block_id() and drops
+// the blocks past the end, of which the last row of the grid may have some.
+constexpr long long GRID_X = 1LL << 22;
+inline dim3 wide_grid(long long blocks) {
+    const long long x = blocks < GRID_X ? blocks : GRID_X;
+    return dim3((unsigned)x, (unsigned)((blocks + x - 1) / x));
+}
+
 inline int launch_check(const char* what) { return hip_check(hipGetLastError(), what); }
 
 // Optional per-kernel timing: a hipEvent pair on the launch stream around every kernel launch while enabled.

@@ -32,6 +32,9 @@ __device__ __forceinline__ long long xcd_logical(long long b, long long nb) {
     return x < r ? x * (q + 1) + s : r * (q + 1) + (x - r) * q + s;
 }
 
+// The block's index in a launch of wide_grid: the second dimension is 1 up to 2^22 blocks.
+__device__ __forceinline__ long long block_id() { return (long long)blockIdx.y * gridDim.x + blockIdx.x; }
+
 // Index of the calling wavefront in its workgroup, as a wave-uniform (scalar) value: everything derived from it
 // (tracer, plane base pointers) stays in scalar registers instead of being recomputed per lane.
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
