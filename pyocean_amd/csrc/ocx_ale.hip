@@ -94,7 +94,7 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     p.notconv = w.notconv;
     p.hist = w.hist;
     p.out = out;
-    const unsigned gb = (unsigned)((face_cols(AX, ny, nx) + 63) / 64);
+    const dim3 gb = wide_grid((face_cols(AX, ny, nx) + 63) / 64);    // 64 columns a workgroup
     {
         ProfScope _ps("ppm_edges", s);
         launch_edges<AX>(h, act, H_PPM_MIN, n, ny, nx, w.e_lo, w.e_hi, s);
@@ -217,7 +217,7 @@ int ocx_transport_velocity_f64(const double* u_new, const double* u_old, const u
     hipStream_t s = static_cast<hipStream_t>(stream);
     ProfScope _ps("transport_velocity", s);
     if (n <= TV_MAX)
-        k_transport_velocity<<<(unsigned)((columns + 63) / 64), 64 * TV_W, (size_t)n * 2 * 64 * sizeof(double), s>>>(
+        k_transport_velocity<<<wide_grid((columns + 63) / 64), 64 * TV_W, (size_t)n * 2 * 64 * sizeof(double), s>>>(
             u_new, u_old, last_wet, w, L, D, theta, theta_bc, n, columns, ut, Q_bt);
     else
         k_transport_velocity_deep<<<blocks_for(columns), BS, 0, s>>>(u_new, u_old, last_wet, w, L, D, theta, theta_bc,

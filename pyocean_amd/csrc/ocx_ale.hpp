@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64 * TV_W) void k_transport_velocity(
     double* s1 = tv_lds;
     double* s0 = tv_lds + (size_t)n * 64;
     const int lane = threadIdx.x & 63, wv = wave_id();
-    const long long p0 = (long long)blockIdx.x * 64 + lane, p = p0 < M ? p0 : M - 1;
+    const long long p0 = block_id() * 64 + lane, p = p0 < M ? p0 : M - 1;
     const bool wet = last_wet[p] != 0;
     double un[TV_L], uo[TV_L], ww[TV_L];
 #pragma unroll
@@ -469,9 +469,9 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_pass(PpmArgs<AX> p, int m) {
     if (!INIT && m > 0 && p.notconv[m - 1] == 0u) return;
     __shared__ double sF[2][PPM_C * 64], sD[2][PPM_C * 64];
     const int lane = threadIdx.x & 63, wv = wave_id();
-    if (INIT && blockIdx.x == 0)
+    if (INIT && block_id() == 0)
         for (int q = threadIdx.x; q < m; q += 64 * PPM_W) p.notconv[q] = 0u;
-    const long long t0 = (long long)blockIdx.x * 64 + lane;
+    const long long t0 = block_id() * 64 + lane;
     const bool in = t0 < p.g.cols();
     const long long t = in ? t0 : p.g.cols() - 1;
     const Column c = column(p, t);
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_bundle(PpmArgs<AX> p, int m,
         if (p.notconv[q] == 0u) return;
     __shared__ double sF[2][PPM_C * 64], sD[2][PPM_C * 64], sS[2][64];
     const int lane = threadIdx.x & 63, wv = wave_id();
-    const long long t0 = (long long)blockIdx.x * 64 + lane;
+    const long long t0 = block_id() * 64 + lane;
     const bool in = t0 < p.g.cols();
     const long long t = in ? t0 : p.g.cols() - 1;
     const Column c = column(p, t);
@@ -587,7 +587,7 @@ template <int AX>
 __global__ __launch_bounds__(64 * PPM_W) void k_ppm_final(PpmArgs<AX> p, int max_iter) {
     __shared__ double sT[2][3][PPM_C * 64];
     const int lane = threadIdx.x & 63, wv = wave_id();
-    const long long t0 = (long long)blockIdx.x * 64 + lane;
+    const long long t0 = block_id() * 64 + lane;
     const bool in = t0 < p.g.cols();
     const long long t = in ? t0 : p.g.cols() - 1;
     const Column c = column(p, t);

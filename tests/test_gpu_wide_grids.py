@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from pyocean_amd import ops
+from pyocean_amd import ale, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +37,41 @@ def test_diffusion_of_many_blocks(gpu, ny, nz, gib, same):
         want = ops.diffuse_h(t, t if same else t.clone(), h[k:e].contiguous(), act, cx, cy, okx, oky,
                              V[k:e].contiguous(), 100.0, 600.0)
         assert torch.equal(got[:, k:e], want), k
+
+
+# four threads a column: from 2^30 columns on, the threads of one dimension no longer count in 32 bits
+def test_transport_velocity_of_many_columns(gpu):
+    print("[gpu case] wide transport velocity", flush=True)
+    _need_memory(60)
+    rows, cols = 1 << 20, 1088
+    g = torch.Generator(device="cuda").manual_seed(2)
+    u = torch.rand(1, rows, cols, device="cuda", dtype=torch.float64, generator=g)
+    wet = torch.ones(rows, cols, dtype=torch.uint8, device="cuda")
+    ut, Qb = ale.transport_velocity(u, u, wet, u, u[0], u[0], 0.6, 0.5)
+    q = rows // 4
+    for a in range(0, rows, q):                        # the columns are independent
+        x = u[:, a:a + q]
+        w0, w1 = ale.transport_velocity(x, x, wet[a:a + q], x, x[0], x[0], 0.6, 0.5)
+        assert torch.equal(ut[:, a:a + q], w0) and torch.equal(Qb[a:a + q], w1), a
+    del u, ut, Qb, wet, x, w0, w1
+    torch.cuda.empty_cache()
+
+
+def test_ppm_transport_of_many_columns(gpu):
+    print("[gpu case] wide ppm transport", flush=True)
+    _need_memory(120)
+    rows, nx = 1 << 20, 1087
+    g = torch.Generator(device="cuda").manual_seed(3)
+    h = 0.5 + torch.rand(1, rows, nx, device="cuda", dtype=torch.float64, generator=g)
+    u = 0.5 + torch.rand(1, rows, nx + 1, device="cuda", dtype=torch.float64, generator=g)
+    act = torch.ones(rows, nx, dtype=torch.uint8, device="cuda")
+    ws = ops.Workspace()
+    call = lambda h, u, act: ale.ppm_transport(h, u, u[0], u[0], u, u, act, 0.1, h[0], 0, 1,        # noqa: E731
+                                               workspace=ws)
+    out = call(h, u, act)
+    q = rows // 4
+    for a in range(0, rows, q):                        # so are the rows, but for the stop of all columns' iterations
+        part = call(h[:, a:a + q], u[:, a:a + q], act[a:a + q])
+        assert torch.equal(out[:, a:a + q], part), a
+    del h, u, act, ws, out, part
+    torch.cuda.empty_cache()
