@@ -6,13 +6,15 @@ holds ``waves_per_group`` wavefronts, one tracer each, over the same strip, chun
 per-cell fields (Qx, Qy, V0, V1, ok) through the L1/L2.  A launch shape is therefore
 
 * ``rows_per_chunk`` - the y extent of one work item (each chunk re-reads a 3-row halo at its ends, so longer
-  chunks move fewer bytes but give fewer work items to spread over 256 compute units);
+  chunks move fewer bytes but give fewer work items to spread over 256 compute units); 0: the untuned shape, whose
+  rows the library chooses by the wavefronts of the call, timed once;
 * ``waves_per_group`` - the lane width of a workgroup, 64 x {1, 2, 4} lanes;
 * ``groups_per_cu`` (batches only) - the persistent grid, in workgroups per compute unit.
 
 The candidates are timed with HIP events on the caller's own workload (every launch shape gives bit-identical
-results, so tuning changes speed only).  Results are cached in a JSON file (``OCX_TUNING_CACHE`` or
-``~/.cache/pyocean_amd/tuning.json``) keyed by device name, precision and shape.
+results, so tuning changes speed only).  The untuned shape is among them, so that a tuned call is not slower than an
+untuned one.  Results are cached in a JSON file (``OCX_TUNING_CACHE`` or ``~/.cache/pyocean_amd/tuning.json``) keyed by
+device name, precision and shape, and by the version of the rules that choose the untuned shape (``RULES``).
 """
 from __future__ import annotations
 
@@ -26,9 +28,11 @@ import torch
 
 from . import batch, ops
 
-ROWS = (16, 32, 64, 128, 256)
+ROWS = (0, 2, 4, 8, 16, 32, 64, 128, 256)
+BATCH_ROWS = (0, 8, 16, 32, 64, 128, 256)      # a batch's work items come from a queue: shorter chunks never gain
 WAVES = (1, 2, 4)
 GROUPS = (1, 2, 4, 8)
+RULES = 2           # goes up with the library's rules for the untuned shape: a cached winner has to have met them
 
 
 @dataclass(frozen=True)
@@ -40,7 +44,9 @@ class Shape:
     @property
     def tile(self) -> str:
         """The work item as (x lanes) x (y rows) x (layers)."""
-        return f"{64 * self.waves_per_group}x{self.rows_per_chunk}x1"
+        if not self.rows_per_chunk:
+            return "untuned"
+        return f"{64 * max(self.waves_per_group, 1)}x{self.rows_per_chunk}x1"
 
 
 def cache_path() -> Path:
@@ -71,12 +77,17 @@ def _store(key: str, shape: Shape) -> None:
 
 def _key(kind: str, precision: str, shapes) -> str:
     dev = torch.cuda.get_device_name(torch.cuda.current_device()).replace(" ", "_")
-    return f"{dev}|{kind}|{precision}|" + ",".join("x".join(str(v) for v in s) for s in shapes)
+    return f"{dev}|{kind}|rules{RULES}|{precision}|" + ",".join("x".join(str(v) for v in s) for s in shapes)
 
 
 def cached(kind: str, precision: str, shapes) -> Shape | None:
     v = _load().get(_key(kind, precision, shapes))
     return Shape(**v) if v else None
+
+
+def _candidates(rows, *others):
+    """The launch shapes to time: the untuned one once where ``rows`` holds 0, and every combination of the rest."""
+    return [(0,) * (1 + len(others))] * (0 in rows) + list(itertools.product([r for r in rows if r], *others))
 
 
 def _time_ms(fn, reps: int, stream) -> float:
@@ -95,7 +106,8 @@ def _time_ms(fn, reps: int, stream) -> float:
 def tune_step(C, V0, V1, Qx, Qy, ok, dt, precision: str = "f64", flags: int = 0, inflow=None, reps: int = 3,
               rows=ROWS, waves=WAVES, use_cache: bool = True, log=None):
     """Tune the single-domain step (``ops.advect_fct``) on these inputs; leaves the best shape set
-    (``batch.set_tuning``) and returns (best, table) with table = [(shape, ms)].  C is not modified."""
+    (``batch.set_tuning``: for every later single-domain call of the process, whatever its size) and returns
+    (best, table) with table = [(shape, ms)].  C is not modified."""
     shapes = [tuple(C.shape)]
     if use_cache:
         hit = cached("step", precision, shapes)
@@ -106,7 +118,7 @@ def tune_step(C, V0, V1, Qx, Qy, ok, dt, precision: str = "f64", flags: int = 0,
     ws = ops.Workspace()
     stream = torch.cuda.current_stream()
     table = []
-    for r, w in itertools.product(rows, waves):
+    for r, w in _candidates(rows, waves):
         batch.set_tuning(r, w)
         ms = _time_ms(lambda: ops.advect_fct(C, V0, V1, Qx, Qy, ok, dt, inflow=inflow, flags=flags, out=out,
                                              workspace=ws, precision=precision), reps, stream)
@@ -119,7 +131,7 @@ def tune_step(C, V0, V1, Qx, Qy, ok, dt, precision: str = "f64", flags: int = 0,
     return best, table
 
 
-def tune_batch(domains: list[batch.Domain], reps: int = 2, rows=ROWS, waves=WAVES, groups=GROUPS,
+def tune_batch(domains: list[batch.Domain], reps: int = 2, rows=BATCH_ROWS, waves=WAVES, groups=GROUPS,
                graph: bool = False, use_cache: bool = True, log=None):
     """Tune the batched step over ``domains``.  Returns (best, table, steps_taken): every trial step advances the
     domains' states (``steps_taken`` steps in all; each launch shape computes the same states, so the domains end
@@ -143,7 +155,7 @@ def tune_batch(domains: list[batch.Domain], reps: int = 2, rows=ROWS, waves=WAVE
         d.C_alt = probe.spare(m)
         d.workspace = probe.workspace(m)
     probe.close()
-    for r, w, g in itertools.product(rows, waves, groups):
+    for r, w, g in _candidates(rows, waves, groups):
         b = batch.Batch(doms, rows_per_chunk=r, waves_per_group=w, groups_per_cu=g)
 
         def two():
