@@ -243,11 +243,14 @@ typedef struct ocx_domain {
 
 typedef struct ocx_batch ocx_batch;
 
-/* rows_per_chunk: rows one wavefront marches (0: 2 .. 64, by the wavefronts the call gives); waves_per_group:
+/* rows_per_chunk: rows one wavefront marches (0: 8 .. 64, by the work of the members together); waves_per_group:
  * wavefronts per workgroup, the tracers of one layer (0: 2, at most 4); groups_per_cu: resident workgroups per compute
- * unit of the persistent grid (0: 4).  Copies the domain table to the device (synchronous). */
+ * unit of the persistent grid (0: as many as fit).  Copies the domain table to the device (synchronous). */
 int ocx_batch_create(const ocx_domain* domains, int ndomains, int rows_per_chunk, int waves_per_group,
                      int groups_per_cu, ocx_batch** out);
+/* The rows per chunk that ocx_batch_create takes for these members (their sizes only) and this waves_per_group with
+ * rows_per_chunk 0, or OCX_E_ARG.  A host computation. */
+int ocx_batch_rows(const ocx_domain* domains, int ndomains, int waves_per_group);
 int ocx_batch_step(ocx_batch* batch, int parity, void* stream);
 /* Captures the step of this parity into a hipGraph on its first call (stream must not be the NULL stream), then
  * launches the graph. */
@@ -255,7 +258,8 @@ int ocx_batch_graph_step(ocx_batch* batch, int parity, void* stream);
 int ocx_batch_destroy(ocx_batch* batch);
 
 /* Launch shape of the single-domain entry points (for the autotuner; no counterpart in the reference):
- * rows_per_chunk and waves_per_group as for ocx_batch_create; 0 restores the default.  Process-wide. */
+ * rows_per_chunk and waves_per_group as for ocx_batch_create; 0 restores the default (2 .. 64 rows by the wavefronts
+ * of each call, one wavefront per workgroup).  Process-wide. */
 int ocx_set_tuning(int rows_per_chunk, int waves_per_group);
 
 /* Per-kernel timing (no counterpart in the reference; for benchmarks): while enabled, every kernel launch of this

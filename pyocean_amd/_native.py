@@ -80,6 +80,7 @@ SIGNATURES = {
     "ocx_freshwater_volumes_f64": (I, [P, P, D, P, D, P, I, I, I, P, P, P, Z, P, P]),
     "ocx_apply_freshwater_f64": (I, [P, I, I, I, I, I, I, I, P, P, P, D, P, P, Z, P, P]),
     "ocx_batch_create": (I, [P, I, I, I, I, P]),
+    "ocx_batch_rows": (I, [P, I, I]),
     "ocx_batch_step": (I, [P, I, P]),
     "ocx_batch_graph_step": (I, [P, I, P]),
     "ocx_batch_destroy": (I, [P]),

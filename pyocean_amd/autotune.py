@@ -32,7 +32,7 @@ ROWS = (0, 2, 4, 8, 16, 32, 64, 128, 256)
 BATCH_ROWS = (0, 8, 16, 32, 64, 128, 256)      # a batch's work items come from a queue: shorter chunks never gain
 WAVES = (1, 2, 4)
 GROUPS = (1, 2, 4, 8)
-RULES = 2           # goes up with the library's rules for the untuned shape: a cached winner has to have met them
+RULES = 3           # goes up with the library's rules for the untuned shape: a cached winner has to have met them
 
 
 @dataclass(frozen=True)

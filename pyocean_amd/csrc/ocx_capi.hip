@@ -150,6 +150,32 @@ long long march_waves(int nt, int nz, int ny, int nx, int r) {
     return (long long)((nx + ocx::MS - 1) / ocx::MS) * ((ny + r - 1) / r) * nt * nz;
 }
 
+// Rows per chunk of a batch, whose members share the launch.  Its workgroups (wpb tracers each) take their chunks from
+// queues, about 0.1 us a chunk and queue, and each looks through all eight queues before it leaves, so chunks as short
+// as a single call's cost more than the chain they shorten; a chunk should also hold about 64 tracer-rows.  So: 64
+// rows where those give 65536 wavefronts (as in a single call) or a workgroup holds one tracer, else 32, and less
+// (to 8) only while the launch has fewer chunks than the chip has compute units.  Measured (us per step, rows 8 / 16 /
+// 32 / 64; FP64, then split), one domain of 96 x 80 x 8 x 2 tracers 136 / 209 / 350 / 602, 115 / 170 / 255 / 416; 16
+// of them 710 / 664 / 607 / 739, 938 / 582 / 487 / 514; 64 of them 1333 / 1213 / 1207 / 1760, 1376 / 1233 / 1271 /
+// 1321; 2 of 300 x 250 x 30 x 4 2017 / 1869 / 1775 / 2037, 1872 / 1673 / 1552 / 1777; one tracer, 198 x 159 x 50, 2
+// domains 1397 / 1336 / 1155 / 1279, 1960 / 1508 / 956 / 926, 8 domains 2555 / 2205 / 2036 / 2167, 3054 / 2517 / 2434 /
+// 2238.  The single call's rule gave these 2 to 16 rows.  Where a domain is one chunk of 64 rows, halves can lose: 64
+// domains of 64 x 64 x 4 x 2 697 / 722 (32 / 64), split 623 / 522.
+int batch_rows(const ocx_domain* dom, int ndom, int wpb) {
+    auto sum = [&](int r, bool chunks) {
+        long long w = 0;
+        for (int d = 0; d < ndom; ++d)
+            w += march_waves(chunks ? (dom[d].nt + wpb - 1) / wpb : dom[d].nt, dom[d].nz, dom[d].ny, dom[d].nx, r);
+        return w;
+    };
+    if (wpb == 1 || sum(MAX_RCH, false) >= 65536) {
+        if (sum(MAX_RCH, true) >= 256) return MAX_RCH;
+    }
+    int r = MAX_RCH / 2;
+    while (r > 8 && sum(r, true) < 256) r /= 2;
+    return r;
+}
+
 int rows_per_chunk(int nt, int nz, int ny, int nx) {
     const int r = g_rch.load();
     return r > 0 ? r : auto_rows([&](int rr) { return march_waves(nt, nz, ny, nx, rr); });
@@ -878,6 +904,18 @@ int ocx_set_tuning(int rows_per_chunk, int waves_per_group) {
     return OCX_OK;
 }
 
+int ocx_batch_rows(const ocx_domain* domains, int ndomains, int waves_per_group) {
+    if (ndomains < 1 || !domains) return fail(OCX_E_ARG, "no domains");
+    if (waves_per_group < 0 || waves_per_group > ocx::MAXW)
+        return fail(OCX_E_ARG, "bad tuning (waves_per_group=%d)", waves_per_group);
+    int maxnt = 1;
+    for (int d = 0; d < ndomains; ++d) {
+        OCX_TRY(check_shape(domains[d].nt, domains[d].nz, domains[d].ny, domains[d].nx));
+        maxnt = std::max(maxnt, domains[d].nt);
+    }
+    return batch_rows(domains, ndomains, tracer_group(maxnt, waves_per_group > 0 ? waves_per_group : DEFAULT_BATCH_WPB));
+}
+
 int ocx_batch_create(const ocx_domain* domains, int ndomains, int rows_per_chunk, int waves_per_group,
                      int groups_per_cu, ocx_batch** out) {
     using namespace ocx;
@@ -892,17 +930,11 @@ int ocx_batch_create(const ocx_domain* domains, int ndomains, int rows_per_chunk
         OCX_TRY(check_shape(domains[d].nt, domains[d].nz, domains[d].ny, domains[d].nx));
         maxnt = std::max(maxnt, domains[d].nt);
     }
-    // rows per chunk by the wavefronts of all members together, which share the launch
-    const int rch = rows_per_chunk > 0 ? rows_per_chunk : auto_rows([&](int r) {
-        long long w = 0;
-        for (int d = 0; d < ndomains; ++d)
-            w += march_waves(domains[d].nt, domains[d].nz, domains[d].ny, domains[d].nx, r);
-        return w;
-    });
     // two tracers per workgroup unless asked otherwise (the 64-domain batch measured 149.5 ms per step with two,
     // 150.7 with one)
     const int wg = waves_per_group > 0 ? waves_per_group : DEFAULT_BATCH_WPB;
     const int wpb = tracer_group(maxnt, wg), wpl = limit_group(maxnt, wg);
+    const int rch = rows_per_chunk > 0 ? rows_per_chunk : batch_rows(domains, ndomains, wpb);
     std::vector<BatchDomain> h(ndomains);
     std::vector<long long> pm(ndomains + 1, 0), pl(ndomains + 1, 0);
     for (int d = 0; d < ndomains; ++d) {

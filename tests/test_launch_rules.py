@@ -1,0 +1,36 @@
+"""
+The launch shapes that a call's size chooses (host computations, no GPU).
+"""
+from __future__ import annotations
+
+import pytest
+
+from pyocean_amd import _native
+from pyocean_amd._native import OcxDomain
+
+
+def _domains(*shapes):
+    d = (OcxDomain * len(shapes))()
+    for q, (nx, ny, nz, nt) in enumerate(shapes):
+        d[q].nx, d[q].ny, d[q].nz, d[q].nt = nx, ny, nz, nt
+    return d
+
+
+BASIN, BAY, COAST = (96, 80, 8, 2), (198, 159, 50, 1), (300, 250, 30, 4)
+
+
+# 64 rows with one tracer a workgroup or a full chip, 32 with two, less while the chip has fewer chunks than units
+@pytest.mark.parametrize("shapes,wpg,rows", [
+    ([BASIN], 0, 8), ([BASIN] * 4, 0, 16), ([BASIN] * 16, 0, 32), ([BASIN] * 64, 0, 32), ([BASIN] * 8, 1, 64),
+    ([BAY], 0, 64), ([BAY] * 2, 0, 64), ([BAY] * 8, 0, 64), ([COAST] * 2, 0, 32), ([COAST] * 2, 1, 64),
+    ([(96, 80, 8, 1)] * 4, 0, 16), ([(96, 80, 8, 1), (198, 159, 50, 3)], 0, 32), ([(1024, 1024, 50, 10)], 0, 64),
+    ([(1, 1, 1, 1)], 0, 8)])
+def test_batch_rows(shapes, wpg, rows):
+    assert _native.lib().ocx_batch_rows(_domains(*shapes), len(shapes), wpg) == rows
+
+
+def test_batch_rows_refuses_what_create_refuses():
+    L = _native.lib()
+    assert L.ocx_batch_rows(_domains((0, 1, 1, 1)), 1, 0) == _native.OCX_E_ARG
+    assert L.ocx_batch_rows(_domains(BASIN), 1, 9) == _native.OCX_E_ARG
+    assert L.ocx_batch_rows(None, 0, 0) == _native.OCX_E_ARG
