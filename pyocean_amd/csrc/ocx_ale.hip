@@ -35,6 +35,13 @@ long long face_cols(int axis, int ny, int nx) {
     return axis == 0 ? (long long)ny * (nx + 1) : (long long)(ny + 1) * nx;
 }
 
+// Newton iterations to a launch after the first PPM_SINGLE, and the iterations with a launch of their own
+// (k_ppm_bundle says why)
+int ppm_bundle_of(int axis, int ny, int nx) {
+    return (int)std::max(1LL, std::min((long long)PPM_BUNDLE, 8192 / ((face_cols(axis, ny, nx) + 63) / 64)));
+}
+int ppm_single_of(int bundle, int max_iter) { return bundle > 1 ? PPM_SINGLE : std::max(max_iter, 1); }
+
 // PPM workspace: the two edge stacks, the Newton state per face column, the convergence flags
 struct PpmWs {
     double *e_lo, *e_hi, *du, *lo, *hi, *err, *dsum, *hist;
@@ -56,7 +63,8 @@ size_t ppm_layout(void* base, int n, int ny, int nx, int axis, int max_iter, Ppm
     t.err = cv.take<double>(cols);
     t.dsum = cv.take<double>(cols);
     t.notconv = cv.take<unsigned>((size_t)std::max(max_iter, 1));
-    t.hist = cv.take<double>(cols * (size_t)std::min(std::max(max_iter - PPM_SINGLE, 0), PPM_BUNDLE));
+    const int bundle = ppm_bundle_of(axis, ny, nx);
+    t.hist = cv.take<double>(cols * (size_t)std::min(std::max(max_iter - ppm_single_of(bundle, max_iter), 0), bundle));
     if (w) *w = t;
     return cv.used;
 }
@@ -94,6 +102,8 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     p.notconv = w.notconv;
     p.hist = w.hist;
     p.out = out;
+    p.bundle = ppm_bundle_of(AX, ny, nx);
+    p.single = ppm_single_of(p.bundle, max_iter);
     const dim3 gb = wide_grid((face_cols(AX, ny, nx) + 63) / 64);    // 64 columns a workgroup
     {
         ProfScope _ps("ppm_edges", s);
@@ -105,13 +115,13 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
         k_ppm_pass<AX, true><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
     }
     OCX_TRY(launch_check("ppm init"));
-    for (int m = 0; m < std::min(max_iter, PPM_SINGLE); ++m) {
+    for (int m = 0; m < std::min(max_iter, p.single); ++m) {
         ProfScope _ps("ppm_newton", s);
         k_ppm_pass<AX, false><<<gb, 64 * PPM_W, 0, s>>>(p, m);
     }
-    for (int m = PPM_SINGLE; m < max_iter; m += PPM_BUNDLE) {
+    for (int m = p.single; m < max_iter; m += p.bundle) {
         ProfScope _ps("ppm_newton_bundle", s);
-        k_ppm_bundle<AX><<<gb, 64 * PPM_W, 0, s>>>(p, m, std::min(PPM_BUNDLE, max_iter - m));
+        k_ppm_bundle<AX><<<gb, 64 * PPM_W, 0, s>>>(p, m, std::min(p.bundle, max_iter - m));
     }
     OCX_TRY(launch_check("ppm newton"));
     {

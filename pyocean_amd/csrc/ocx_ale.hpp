@@ -325,8 +325,9 @@ struct PpmArgs {
     Geo<AX> g;
     double *du, *lo, *hi, *err, *dsum;   // state per face column
     unsigned* notconv;                   // notconv[m]: some column unconverged after iteration m
-    double* hist;                        // du after each iteration of the last bundle (k_ppm_bundle), PPM_BUNDLE x columns
+    double* hist;                        // du after each iteration of the last bundle (k_ppm_bundle), bundle x columns
     double* out;
+    int single, bundle;                  // iterations with a launch of their own, and iterations in each launch after those
 };
 
 // the face column's geometry: donor cells on both sides and their widths
@@ -537,18 +538,21 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_pass(PpmArgs<AX> p, int m) {
     }
 }
 
-// The iterations m .. m + count - 1 (count <= PPM_BUNDLE) in one launch, without a look at the other columns in between:
-// du after each of them goes to hist, so that the fluxes can take the one after which all columns had converged.  Only
-// the first PPM_SINGLE iterations have launches of their own: 4 to 6 converge every column of the grids measured, and a
-// launch with nothing to do costs 2 to 5 us.  The rest are bundled: of the usual 20 iterations' launches 9 are left per
-// direction, which takes 799 us to 716 for a transport of 198 x 159 x 50 and 0.1 ms off one of 384 x 384 x 50.
-// A bundle in which all columns converge early has iterated on for nothing, at most PPM_BUNDLE - 1 times.
+// The iterations m .. m + count - 1 (count <= p.bundle) in one launch, without a look at the other columns in between:
+// du after each of them goes to hist, so that the fluxes can take the one after which all columns had converged.  4 to
+// 6 iterations converge every column of the grids measured, and a launch with nothing to do costs 2 to 5 us, so of the
+// usual 20 iterations only the first PPM_SINGLE have launches of their own: 799 us to 716 for a transport of 198 x 159
+// x 50 with the other 12 in one bundle.  But a bundle in which all columns converge has iterated on for nothing, up to
+// bundle - 1 times, and from some 1000 workgroups on that costs more than the launches: a field of 512 x 512 x 50 that
+// takes 9 iterations took 2.59 ms a direction with a bundle of 12, and 1.71 before the layers were shared.  So a bundle
+// has at most PPM_BUNDLE iterations and at most 8192 workgroup-iterations (ppm_bundle_of), and above 4096 workgroups
+// every iteration has a launch of its own.
 constexpr int PPM_SINGLE = 8, PPM_BUNDLE = 12;
 template <int AX>
 __global__ __launch_bounds__(64 * PPM_W) void k_ppm_bundle(PpmArgs<AX> p, int m, int count) {
     // nothing to do once an iteration before this bundle has converged everywhere (flags of iterations that were not
     // run are 0 too)
-    for (int q = m > PPM_SINGLE ? m - PPM_BUNDLE : m - 1; q < m; ++q)
+    for (int q = m > p.single ? m - p.bundle : m - 1; q < m; ++q)
         if (p.notconv[q] == 0u) return;
     __shared__ double sF[2][PPM_C * 64], sD[2][PPM_C * 64], sS[2][64];
     const int lane = threadIdx.x & 63, wv = wave_id();
@@ -597,7 +601,7 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_final(PpmArgs<AX> p, int max
     // the first iteration after which every column had converged, or the last
     int it = 0;
     while (it < max_iter - 1 && p.notconv[it] != 0u) ++it;
-    const double du = it < PPM_SINGLE ? p.du[t] : p.hist[(size_t)((it - PPM_SINGLE) % PPM_BUNDLE) * p.g.cols() + t];
+    const double du = it < p.single ? p.du[t] : p.hist[(size_t)((it - p.single) % p.bundle) * p.g.cols() + t];
     double sum = 0.0;                       // wavefront 0: of F, 1: of q_e, 2: of q_w
     for (int kc = 0, b = 0; kc < n; kc += PPM_C, b ^= 1) {
         const int k = kc + wv * PPM_L;

@@ -141,3 +141,21 @@ def test_limit_outflow_keeps_the_fluxes_of_the_error(gpu, n, axis):
         assert tuple(where)[1:] == face
         _bits(dy, want[1], "Qy")
     assert not np.array_equal(dx.cpu().numpy() if axis == 0 else dy.cpu().numpy(), want[axis])
+
+
+# grids whose bundles hold 12, 5, 2 and (every iteration alone) 1 iterations
+@pytest.mark.parametrize("max_iter", [9, 11, 20])
+@pytest.mark.parametrize("nx,ny", [(40, 13), (310, 316), (500, 440), (530, 520)])
+def test_bundles_of_every_length_stop_where_the_oracle_stops(gpu, nx, ny, max_iter):
+    print("[gpu case] bundle lengths", nx, ny, max_iter, flush=True)
+    a = synth.ale_inputs(nx, ny, 2, seed=4)
+    act = np.asarray(a.active, bool)
+    ut, Qb = R.transport_velocity(a.u_new, a.u_old, a.wet_u, a.wu, a.Lu, a.Du, a.theta, a.theta_bc)
+    qe, qw = R.face_transport_thickness(a.h, a.H, act, True)
+    for reach in (1.0, 50.0):                 # converges after a few iterations; never
+        want, rit = R.ppm_transport_x(a.h, ut, a.Lu, Qb * reach, qe, qw, act, a.dt, a.dx_t, max_iter,
+                                      return_iterations=True)
+        got, it = ale.ppm_transport(_d(a.h), _d(ut), _d(a.Lu), _d(Qb * reach), _d(qe), _d(qw), _d(act), a.dt, _d(a.dx_t),
+                                    0, max_iter, return_iterations=True)
+        assert it == rit
+        _bits(got, want, "Q")

@@ -34,3 +34,13 @@ def test_batch_rows_refuses_what_create_refuses():
     assert L.ocx_batch_rows(_domains((0, 1, 1, 1)), 1, 0) == _native.OCX_E_ARG
     assert L.ocx_batch_rows(_domains(BASIN), 1, 9) == _native.OCX_E_ARG
     assert L.ocx_batch_rows(None, 0, 0) == _native.OCX_E_ARG
+
+
+# the history of bundled iterations costs a large grid nothing: every iteration has a launch of its own there
+@pytest.mark.parametrize("nx,ny,columns", [(197, 159, 12), (384, 383, 3), (511, 513, 0), (1024, 1024, 0)])
+def test_ppm_workspace_holds_the_history_of_one_bundle(nx, ny, columns):
+    L = _native.lib()
+    for axis, cols in ((0, ny * (nx + 1)), (1, (ny + 1) * nx)):
+        size = [int(L.ocx_ppm_transport_workspace_bytes(50, ny, nx, axis, m)) for m in (8, 20)]
+        want = columns * cols * 8
+        assert abs(size[1] - size[0] - want) <= 512
