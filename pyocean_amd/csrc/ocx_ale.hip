@@ -42,6 +42,18 @@ int ppm_bundle_of(int axis, int ny, int nx) {
 }
 int ppm_single_of(int bundle, int max_iter) { return bundle > 1 ? PPM_SINGLE : std::max(max_iter, 1); }
 
+// Whether a thread takes a whole face column (k_ppm_walk) instead of a workgroup's wavefronts sharing its layers
+// (k_ppm_pass).  Sharing takes chunks of PPM_C layers, so short columns leave wavefronts without a layer, and once the
+// grid fills the chip by itself (above 4096 workgroups of 64 columns) a chunk that is mostly empty costs as much as it
+// saves.  So: walked up to 5 layers, and on such grids where a quarter of the chunks' layers or more are beyond the
+// column.  Measured (us a direction, shared / walked): 384 x 384 3 layers 185 / 131, 6 178 / 162, 12 211 / 213, 50 599 /
+// 622; 1024 x 1024 1 layer 900 / 559, 8 1264 / 1070, 12 1514 / 1390, 16 1725 / 1744, 20 2189 / 2014, 33 2903 / 2780, 41
+// 3383 / 3466, 50 4170 / 4200; 2000 x 2000 1 layer 3579 / 2088, 10 4923 / 4477.
+bool ppm_walks(int axis, int n, int ny, int nx) {
+    const int slots = (n + PPM_C - 1) / PPM_C * PPM_C;
+    return n <= 5 || ((face_cols(axis, ny, nx) + 63) / 64 > 4096 && 4LL * n <= 3LL * slots);
+}
+
 // PPM workspace: the two edge stacks, the Newton state per face column, the convergence flags
 struct PpmWs {
     double *e_lo, *e_hi, *du, *lo, *hi, *err, *dsum, *hist;
@@ -105,6 +117,8 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     p.bundle = ppm_bundle_of(AX, ny, nx);
     p.single = ppm_single_of(p.bundle, max_iter);
     const dim3 gb = wide_grid((face_cols(AX, ny, nx) + 63) / 64);    // 64 columns a workgroup
+    const unsigned wb = blocks_for(face_cols(AX, ny, nx));
+    const bool walk = ppm_walks(AX, n, ny, nx);
     {
         ProfScope _ps("ppm_edges", s);
         launch_edges<AX>(h, act, H_PPM_MIN, n, ny, nx, w.e_lo, w.e_hi, s);
@@ -112,12 +126,18 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     OCX_TRY(launch_check("ppm edges"));
     {
         ProfScope _ps("ppm_init", s);
-        k_ppm_pass<AX, true><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
+        if (walk)
+            k_ppm_walk<AX, true><<<wb, BS, 0, s>>>(p, max_iter);
+        else
+            k_ppm_pass<AX, true><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
     }
     OCX_TRY(launch_check("ppm init"));
     for (int m = 0; m < std::min(max_iter, p.single); ++m) {
         ProfScope _ps("ppm_newton", s);
-        k_ppm_pass<AX, false><<<gb, 64 * PPM_W, 0, s>>>(p, m);
+        if (walk)
+            k_ppm_walk<AX, false><<<wb, BS, 0, s>>>(p, m);
+        else
+            k_ppm_pass<AX, false><<<gb, 64 * PPM_W, 0, s>>>(p, m);
     }
     for (int m = p.single; m < max_iter; m += p.bundle) {
         ProfScope _ps("ppm_newton_bundle", s);
@@ -126,7 +146,10 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     OCX_TRY(launch_check("ppm newton"));
     {
         ProfScope _ps("ppm_final", s);
-        k_ppm_final<AX><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
+        if (walk)
+            k_ppm_walk_final<AX><<<wb, BS, 0, s>>>(p, max_iter);
+        else
+            k_ppm_final<AX><<<gb, 64 * PPM_W, 0, s>>>(p, max_iter);
     }
     return launch_check("ppm final");
 }

@@ -16,6 +16,8 @@
 #pragma once
 #include <float.h>
 
+#include <type_traits>
+
 #include "ocx_weno.hpp"
 
 namespace ocx {
@@ -366,16 +368,16 @@ __device__ __forceinline__ Column column(const PpmArgs<AX>& p, long long t) {
 // and 155 -> 106; 1024 x 1024 x 50, where both stream, the whole transport 14.3 -> 12.4 ms).
 constexpr int PPM_W = 4, PPM_L = 4, PPM_C = PPM_W * PPM_L;
 
-// terms of the layers k .. k + PPM_L - 1 (beyond n: repeated, not added): F and dF/du at velocity u^theta + du: the
+// terms of the layers k .. k + NL - 1 (beyond n: repeated, not added): F and dF/du at velocity u^theta + du: the
 // swept mean thickness of the donor parabola over the Courant fraction, capped by the transport thickness where that
 // is below the donor layer.  u: the velocities u^theta of these layers.
-template <int AX>
+template <int AX, int NL = PPM_L>
 __device__ __forceinline__ void layer_fluxes(const PpmArgs<AX>& p, const Column& c, int k, const double* u, double* F,
                                              double* dF) {
     const size_t PC = p.g.pc(), PF = p.g.pf();
-    double hu[PPM_L], ww[PPM_L], ee[PPM_L], qq[PPM_L];
+    double hu[NL], ww[NL], ee[NL], qq[NL];
 #pragma unroll
-    for (int q = 0; q < PPM_L; ++q) {
+    for (int q = 0; q < NL; ++q) {
         const size_t kk = (size_t)min(k + q, p.g.n - 1);
         const bool pos = u[q] >= 0.0;
         const size_t ci = kk * PC + (pos ? c.cw : c.ce);
@@ -385,7 +387,7 @@ __device__ __forceinline__ void layer_fluxes(const PpmArgs<AX>& p, const Column&
         qq[q] = (pos ? p.qe : p.qw)[kk * PF + c.fo];
     }
 #pragma unroll
-    for (int q = 0; q < PPM_L; ++q) {
+    for (int q = 0; q < NL; ++q) {
         const bool pos = u[q] >= 0.0;
         const double cr = amin(qdiv_r(fabs(u[q]) * p.dt, pos ? c.rw : c.re), 1.0);
         const double h0 = nan0(hu[q]);
@@ -538,6 +540,69 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_pass(PpmArgs<AX> p, int m) {
     }
 }
 
+// The same with all layers of a column in one thread, PPM_L of them in flight, then the rest one by one, for short
+// columns and for grids that fill the chip (ppm_walks has the line and both sides); state and results as k_ppm_pass.
+template <int AX, bool INIT>
+__global__ __launch_bounds__(256) void k_ppm_walk(PpmArgs<AX> p, int m) {
+    if (!INIT && m > 0 && p.notconv[m - 1] == 0u) return;
+    const long long t = gtid();
+    if (INIT && blockIdx.x == 0)
+        for (int q = threadIdx.x; q < m; q += 256) p.notconv[q] = 0u;
+    bool bad = false;
+    if (t < p.g.cols()) {
+        const Column c = column(p, t);
+        const size_t PF = p.g.pf();
+        const int n = p.g.n;
+        const double limw = 0.5 * c.dxw / p.dt, lime = 0.5 * c.dxe / p.dt;
+        double mnw = __builtin_inf(), mxe = -__builtin_inf();
+        Newton s{0.0, 0.0, 0.0, 0.0, 0.0};
+        if constexpr (!INIT) {
+            s = Newton{p.du[t], p.lo[t], p.hi[t], p.err[t], p.dsum[t]};
+            newton_step(s);
+        }
+        double sum = 0.0, dsum = 0.0;
+        auto layers = [&](auto count, int k) {
+            constexpr int NL = decltype(count)::value;
+            double u[NL], F[NL], dF[NL];
+#pragma unroll
+            for (int q = 0; q < NL; ++q) u[q] = p.ut[(size_t)(k + q) * PF + c.fo];
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+                if constexpr (INIT) {
+                    mnw = amin(mnw, limw - u[q]);
+                    mxe = amax(mxe, -(lime + u[q]));
+                } else {
+                    u[q] = u[q] + s.du;
+                }
+            }
+            if (!c.open) return;
+            layer_fluxes<AX, NL>(p, c, k, u, F, dF);
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+                sum += F[q];
+                dsum += dF[q];
+            }
+        };
+        if (INIT || c.open) {
+            int k = 0;
+            for (; k + PPM_L <= n; k += PPM_L) layers(std::integral_constant<int, PPM_L>{}, k);
+            for (; k < n; ++k) layers(std::integral_constant<int, 1>{}, k);
+        }
+        if constexpr (INIT) {
+            s.hi = amax(amin(limw, mnw), 0.0);
+            s.lo = amin(amax(-lime, mxe), 0.0);
+        }
+        const double er = sum - c.Qb;
+        p.du[t] = s.du;
+        p.hi[t] = s.hi;
+        p.lo[t] = s.lo;
+        p.err[t] = er;
+        p.dsum[t] = dsum;
+        bad = fabs(er) > 1e-12 * amax(fabs(c.Qb), 1.0);
+    }
+    if constexpr (!INIT) wave_flag(bad, p.notconv + m);
+}
+
 // The iterations m .. m + count - 1 (count <= p.bundle) in one launch, without a look at the other columns in between:
 // du after each of them goes to hist, so that the fluxes can take the one after which all columns had converged.  4 to
 // 6 iterations converge every column of the grids measured, and a launch with nothing to do costs 2 to 5 us, so of the
@@ -583,10 +648,31 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_bundle(PpmArgs<AX> p, int m,
     }
 }
 
+// du after the first iteration after which every column had converged, or the last: the state's, or the history's if a
+// bundle converged before its end
+template <int AX>
+__device__ __forceinline__ double final_du(const PpmArgs<AX>& p, long long t, int max_iter) {
+    int it = 0;
+    while (it < max_iter - 1 && p.notconv[it] != 0u) ++it;
+    return it < p.single ? p.du[t] : p.hist[(size_t)((it - p.single) % p.bundle) * p.g.cols() + t];
+}
+
+// the residual's side: its thicknesses and their sum (1 where no side has any)
+template <int AX>
+__device__ __forceinline__ const double* residual_side(const PpmArgs<AX>& p, double R, double te, double tw, Recip& den) {
+    bool use_e = R >= 0.0;
+    double tot = use_e ? te : tw;
+    if (tot <= 0.0) {
+        use_e = !use_e;
+        tot = use_e ? te : tw;
+    }
+    den = recip_of(tot > 0.0 ? tot : 1.0);
+    return use_e ? p.qe : p.qw;
+}
+
 // the layer fluxes at u^theta + du plus the residual R = Q_bt - sum F shared in proportion to the transport thickness
 // on R's side (the other side's where that column is empty); closed faces 0.  The layers are shared by the wavefronts
-// as in k_ppm_pass; the sums of F, q_e and q_w are added by one wavefront each.
-// max_iter: the iterations allowed; du is the state's, or the history's if a bundle converged before its end.
+// as in k_ppm_pass; the sums of F, q_e and q_w are added by one wavefront each.  max_iter: the iterations allowed.
 template <int AX>
 __global__ __launch_bounds__(64 * PPM_W) void k_ppm_final(PpmArgs<AX> p, int max_iter) {
     __shared__ double sT[2][3][PPM_C * 64];
@@ -598,10 +684,7 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_final(PpmArgs<AX> p, int max
     const size_t PF = p.g.pf();
     const int n = p.g.n;
     const bool run = in && c.open;
-    // the first iteration after which every column had converged, or the last
-    int it = 0;
-    while (it < max_iter - 1 && p.notconv[it] != 0u) ++it;
-    const double du = it < p.single ? p.du[t] : p.hist[(size_t)((it - p.single) % p.bundle) * p.g.cols() + t];
+    const double du = final_du(p, t, max_iter);
     double sum = 0.0;                       // wavefront 0: of F, 1: of q_e, 2: of q_w
     for (int kc = 0, b = 0; kc < n; kc += PPM_C, b ^= 1) {
         const int k = kc + wv * PPM_L;
@@ -638,14 +721,8 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_final(PpmArgs<AX> p, int max
     __syncthreads();
     if (!run) return;
     const double R = c.Qb - sT[0][0][lane], te = sT[0][1][lane], tw = sT[0][2][lane];
-    bool use_e = R >= 0.0;
-    double tot = use_e ? te : tw;
-    if (tot <= 0.0) {
-        use_e = !use_e;
-        tot = use_e ? te : tw;
-    }
-    const Recip den = recip_of(tot > 0.0 ? tot : 1.0);
-    const double* q = use_e ? p.qe : p.qw;
+    Recip den;
+    const double* q = residual_side(p, R, te, tw, den);
     for (int kc = wv * PPM_L; kc < n; kc += PPM_C) {
         double f[PPM_L], qk[PPM_L];
 #pragma unroll
@@ -657,6 +734,53 @@ __global__ __launch_bounds__(64 * PPM_W) void k_ppm_final(PpmArgs<AX> p, int max
 #pragma unroll
         for (int l = 0; l < PPM_L; ++l)
             if (kc + l < n) p.out[(size_t)(kc + l) * PF + c.fo] = f[l] + qdiv_r(R * qk[l], den);
+    }
+}
+
+// The same with all layers of a column in one thread.
+template <int AX>
+__global__ __launch_bounds__(256) void k_ppm_walk_final(PpmArgs<AX> p, int max_iter) {
+    const long long t = gtid();
+    if (t >= p.g.cols()) return;
+    const Column c = column(p, t);
+    const size_t PF = p.g.pf();
+    const int n = p.g.n;
+    if (!c.open) {
+        for (int k = 0; k < n; ++k) p.out[(size_t)k * PF + c.fo] = 0.0;
+        return;
+    }
+    const double du = final_du(p, t, max_iter);
+    double sum = 0.0, te = 0.0, tw = 0.0;
+    auto layers = [&](auto count, int k) {
+        constexpr int NL = decltype(count)::value;
+        double u[NL], F[NL], dF[NL], qe[NL], qw[NL];
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const size_t x = (size_t)(k + q) * PF + c.fo;
+            u[q] = p.ut[x];
+            qe[q] = p.qe[x];
+            qw[q] = p.qw[x];
+        }
+#pragma unroll
+        for (int q = 0; q < NL; ++q) u[q] = u[q] + du;
+        layer_fluxes<AX, NL>(p, c, k, u, F, dF);
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            p.out[(size_t)(k + q) * PF + c.fo] = F[q];
+            sum += F[q];
+            te += qe[q];
+            tw += qw[q];
+        }
+    };
+    int k = 0;
+    for (; k + PPM_L <= n; k += PPM_L) layers(std::integral_constant<int, PPM_L>{}, k);
+    for (; k < n; ++k) layers(std::integral_constant<int, 1>{}, k);
+    const double R = c.Qb - sum;
+    Recip den;
+    const double* q = residual_side(p, R, te, tw, den);
+    for (k = 0; k < n; ++k) {
+        const size_t x = (size_t)k * PF + c.fo;
+        p.out[x] = p.out[x] + qdiv_r(R * q[x], den);
     }
 }
 

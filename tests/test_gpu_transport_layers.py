@@ -159,3 +159,26 @@ def test_bundles_of_every_length_stop_where_the_oracle_stops(gpu, nx, ny, max_it
                                     0, max_iter, return_iterations=True)
         assert it == rit
         _bits(got, want, "Q")
+
+
+# layer counts on both sides of the line between columns of one thread and columns of a workgroup, on a grid below and
+# on one above the 4096 workgroups at which it moves, with a stop after a few iterations and with none
+@pytest.mark.parametrize("nx,ny,nz", [(63, 40, 1), (63, 40, 4), (63, 40, 5), (63, 40, 6), (530, 520, 5), (530, 520, 11),
+                                      (530, 520, 12), (530, 520, 13), (530, 520, 17)])
+@pytest.mark.parametrize("axis", [0, 1])
+def test_walked_and_shared_columns_match_the_oracle(gpu, nx, ny, nz, axis):
+    print("[gpu case] walked columns", nx, ny, nz, axis, flush=True)
+    a = synth.ale_inputs(nx, ny, nz, seed=6)
+    act = np.asarray(a.active, bool)
+    u1, u0, wet, w, Lf, D, d = ((a.u_new, a.u_old, a.wet_u, a.wu, a.Lu, a.Du, a.dx_t) if axis == 0 else
+                                (a.v_new, a.v_old, a.wet_v, a.wv, a.Lv, a.Dv, a.dy_t))
+    ut, Qb = R.transport_velocity(u1, u0, wet, w, Lf, D, a.theta, a.theta_bc)
+    qp, qn = ale.face_thickness_axis(_d(a.h), _d(a.H), _d(act), True, axis)
+    sw = (lambda x: x) if axis == 0 else (lambda x: np.ascontiguousarray(np.swapaxes(x, -1, -2)))
+    for reach, max_iter in ((1.0, 20), (50.0, 3)):
+        want, rit = R.ppm_transport_x(sw(a.h), sw(ut), sw(Lf), sw(Qb * reach), sw(qp.cpu().numpy()),
+                                      sw(qn.cpu().numpy()), sw(act), a.dt, sw(d), max_iter, return_iterations=True)
+        got, it = ale.ppm_transport(_d(a.h), _d(ut), _d(Lf), _d(Qb * reach), qp, qn, _d(act), a.dt, _d(d), axis, max_iter,
+                                    return_iterations=True)
+        assert it == rit
+        _bits(got, sw(want), f"Q reach {reach}")
