@@ -249,11 +249,11 @@ int ocx_transport_velocity_f64(const double* u_new, const double* u_old, const u
     for (int q = 0; q < 8; ++q) OCX_TRY(need(p[q], nm[q]));
     hipStream_t s = static_cast<hipStream_t>(stream);
     ProfScope _ps("transport_velocity", s);
-    if (n <= TV_MAX)
+    if (n >= TV_MIN && n <= TV_MAX)
         k_transport_velocity<<<wide_grid((columns + 63) / 64), 64 * TV_W, (size_t)n * 2 * 64 * sizeof(double), s>>>(
             u_new, u_old, last_wet, w, L, D, theta, theta_bc, n, columns, ut, Q_bt);
     else
-        k_transport_velocity_deep<<<blocks_for(columns), BS, 0, s>>>(u_new, u_old, last_wet, w, L, D, theta, theta_bc,
+        k_transport_velocity_walk<<<blocks_for(columns), BS, 0, s>>>(u_new, u_old, last_wet, w, L, D, theta, theta_bc,
                                                                      n, columns, ut, Q_bt);
     return launch_check("transport_velocity");
 }

@@ -92,15 +92,17 @@ __device__ __forceinline__ void wave_flag(bool bad, unsigned* flag) {
 }
 
 // ------------------------------------------------------------------------------------------ transport velocity
-// u (n, M) columns; last_wet (M) bytes; w (n, M); L, D (M).  ut (n, M), Qb (M).  Columns of up to TV_MAX layers.
+// u (n, M) columns; last_wet (M) bytes; w (n, M); L, D (M).  ut (n, M), Qb (M).  Columns of TV_MIN to TV_MAX layers.
 //
 // A workgroup holds 64 columns; its TV_W wavefronts share the layers, every one of them TV_L layers in registers, all
 // loads in flight together, so that the column is read once (32 B a cell-layer with the result; a thread that walks
 // its column twice fetched 54) and a small grid does not wait at every layer.  The sums run from the bed up as the
 // reference adds: the products go to LDS as [layer][column] and one wavefront per sum adds them in order.  Layers
 // w, w + TV_W, ... belong to wavefront w.  Dynamic LDS: 2 n * 64 doubles.  198 x 159 x 50 42 -> 17 us a direction,
-// 384 x 384 x 50 79 -> 72.
-constexpr int TV_W = 4, TV_L = 16, TV_MAX = TV_W * TV_L;
+// 384 x 384 x 50 79 -> 72.  Below TV_MIN layers the wavefronts have too little to share (us, shared / one thread a column:
+// 1024 x 1024 1 layer 36 / 16, 3 layers 39 / 24, 5 48 / 45, 8 74 / 70, 10 89 / 87, 12 95 / 112, 20 145 / 202; 2000 x 2000
+// 1 layer 127 / 34, 8 274 / 260, 10 309 / 327; grids up to 384 x 384 are level below 12 layers).
+constexpr int TV_W = 4, TV_L = 16, TV_MIN = 10, TV_MAX = TV_W * TV_L;
 __global__ __launch_bounds__(64 * TV_W) void k_transport_velocity(
     const double* __restrict__ u_new, const double* __restrict__ u_old, const uint8_t* __restrict__ last_wet,
     const double* __restrict__ w, const double* __restrict__ L, const double* __restrict__ D, double theta,
@@ -158,8 +160,8 @@ __global__ __launch_bounds__(64 * TV_W) void k_transport_velocity(
     Qb[p] = L[p] * D[p] * s;
 }
 
-// The same for deeper columns: one thread per column, two walks over its layers.
-__global__ void k_transport_velocity_deep(const double* __restrict__ u_new, const double* __restrict__ u_old,
+// The same for shorter and deeper columns: one thread per column, two walks over its layers.
+__global__ void k_transport_velocity_walk(const double* __restrict__ u_new, const double* __restrict__ u_old,
                                           const uint8_t* __restrict__ last_wet, const double* __restrict__ w,
                                           const double* __restrict__ L, const double* __restrict__ D, double theta,
                                           double theta_bc, int n, long long M, double* __restrict__ ut,

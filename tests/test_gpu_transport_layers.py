@@ -182,3 +182,17 @@ def test_walked_and_shared_columns_match_the_oracle(gpu, nx, ny, nz, axis):
                                     return_iterations=True)
         assert it == rit
         _bits(got, sw(want), f"Q reach {reach}")
+
+
+# the transport velocity's columns of one thread below 10 and above 64 layers
+@pytest.mark.parametrize("n", [1, 2, 9, 10, 11, 64, 65])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (63, 5), (300, 41)])
+def test_transport_velocity_on_both_sides_of_its_lines(gpu, nx, ny, n):
+    print("[gpu case] transport velocity", nx, ny, n, flush=True)
+    rng = np.random.default_rng(n)
+    u1, u0, w = (rng.normal(0, 0.3, (n, ny, nx)) for _ in range(3))
+    wet, Lf, D = rng.random((ny, nx)) > 0.2, rng.uniform(900, 1100, (ny, nx)), rng.uniform(1, 50, (ny, nx))
+    ut, Qb = ale.transport_velocity(_d(u1), _d(u0), _d(wet), _d(w), _d(Lf), _d(D), 0.6, 0.5)
+    rut, rQb = R.transport_velocity(u1, u0, wet, w, Lf, D, 0.6, 0.5)
+    _bits(ut, rut, "ut")
+    _bits(Qb, rQb, "Q_bt")
