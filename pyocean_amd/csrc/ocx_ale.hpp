@@ -988,7 +988,6 @@ struct OutArgs {
     double *r, *room;                    // (n, ny, nx)
     double* delta;                       // per face column of the current axis
     unsigned long long* count;           // cell-layers over the bound
-    unsigned* any;                       // some cell-layer over the bound
     unsigned* wild;                      // some cell-layer's room0 is not finite
     unsigned long long* bad_face;        // first face of the current axis whose cut cannot be given back (linear
                                          // index), else ~0; bad_face[-1]: the u-faces' while the v-faces run
@@ -1014,7 +1013,7 @@ __device__ __forceinline__ double outflow(const OutArgs& o, int k, int j, int i)
     return amax(o.Qx[fx + 1], 0.0) - amin(o.Qx[fx], 0.0) + amax(o.Qy[fy + o.nx], 0.0) - amin(o.Qy[fy], 0.0);
 }
 
-// over = active & O > room0 x factor; r = room0 / O where over, else 1; counts and flags the cells over
+// over = active & O > room0 x factor; r = room0 / O where over, else 1; counts the cells over
 __global__ void k_out_over(OutArgs o, double factor, int first) {
     const long long t = gtid();
     const size_t PC = (size_t)o.ny * o.nx;
@@ -1031,10 +1030,8 @@ __global__ void k_out_over(OutArgs o, double factor, int first) {
     }
     wave_flag(wild, o.wild);
     const unsigned long long b = __ballot(over);
-    if (b && (threadIdx.x & 63) == (unsigned)(__ffsll((long long)b) - 1)) {
+    if (b && (threadIdx.x & 63) == (unsigned)(__ffsll((long long)b) - 1))
         atomicAdd(o.count, (unsigned long long)__popcll(b));
-        atomicOr(o.any, 1u);
-    }
 }
 
 // room = room0 - outflow with the current Qx, Qy
