@@ -273,10 +273,14 @@ int ocx_face_transport_thickness_f64(const double* h, const double* H, const uin
     hipStream_t s = static_cast<hipStream_t>(stream);
     const unsigned gb = blocks_for(face_cols(axis, ny, nx));
     ProfScope _ps("face_thickness", s);
-    if (axis == 0)
-        k_face_thickness<0><<<gb, BS, 0, s>>>(h, H, active, clip, Geo<0>{n, ny, nx}, q_pos, q_neg);
+    const Geo<0> g0{n, ny, nx};
+    const Geo<1> g1{n, ny, nx};
+    if (n < KB / 2)
+        axis == 0 ? k_face_thickness<0, 1><<<gb, BS, 0, s>>>(h, H, active, clip, g0, q_pos, q_neg)
+                  : k_face_thickness<1, 1><<<gb, BS, 0, s>>>(h, H, active, clip, g1, q_pos, q_neg);
     else
-        k_face_thickness<1><<<gb, BS, 0, s>>>(h, H, active, clip, Geo<1>{n, ny, nx}, q_pos, q_neg);
+        axis == 0 ? k_face_thickness<0, KB><<<gb, BS, 0, s>>>(h, H, active, clip, g0, q_pos, q_neg)
+                  : k_face_thickness<1, KB><<<gb, BS, 0, s>>>(h, H, active, clip, g1, q_pos, q_neg);
     return launch_check("face_transport_thickness");
 }
 

@@ -192,7 +192,10 @@ __global__ void k_transport_velocity_walk(const double* __restrict__ u_new, cons
 // ------------------------------------------------------------------------------------------ transport thickness
 // q_e: from the low-side cell (flow towards +), q_w: from the high-side cell; the domain-edge faces use the inner
 // cell, closed faces are 0.  clip: only the part of the donor layer above the shallower bed passes.
-template <int AX>
+// NB layers' loads are in flight, the last one repeated beyond n: KB, and 1 (fewer registers) below KB / 2 layers (us, 1
+// / KB: 2000 x 2000 1 layer 25 / 44, 3 layers 74 / 98, 4 103 / 112, 5 156 / 123, 8 304 / 215; 1024 x 1024 2 layers 14 /
+// 18, 4 22 / 22, 8 54 / 44, 50 771 / 647; 198 x 159 x 50 23 / 18; up to 600 x 600 level below 5 layers).
+template <int AX, int NB>
 __global__ void k_face_thickness(const double* __restrict__ h, const double* __restrict__ H,
                                  const uint8_t* __restrict__ act, int clip, Geo<AX> g, double* __restrict__ qe,
                                  double* __restrict__ qw) {
@@ -216,16 +219,16 @@ __global__ void k_face_thickness(const double* __restrict__ h, const double* __r
         He = He == He ? He : 0.0;
         const double z_bed = amax(-Hw, -He);
         double sw = 0.0, se = 0.0;
-        for (int k = 0; k < g.n; k += KB) {
-            double hw[KB], he[KB];
+        for (int k = 0; k < g.n; k += NB) {
+            double hw[NB], he[NB];
 #pragma unroll
-            for (int q = 0; q < KB; ++q) {
+            for (int q = 0; q < NB; ++q) {
                 const size_t x = (size_t)min(k + q, g.n - 1) * PC;
                 hw[q] = h[x + cw];
                 he[q] = h[x + ce];
             }
 #pragma unroll
-            for (int q = 0; q < KB; ++q) {
+            for (int q = 0; q < NB; ++q) {
                 if (k + q < g.n) {
                     const double a0 = hw[q] == hw[q] ? hw[q] : 0.0, a1 = he[q] == he[q] ? he[q] : 0.0;
                     sw += a0;

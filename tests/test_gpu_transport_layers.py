@@ -196,3 +196,20 @@ def test_transport_velocity_on_both_sides_of_its_lines(gpu, nx, ny, n):
     rut, rQb = R.transport_velocity(u1, u0, wet, w, Lf, D, 0.6, 0.5)
     _bits(ut, rut, "ut")
     _bits(Qb, rQb, "Q_bt")
+
+
+# the transport thicknesses of few layers, taken one by one, and of more, KB = 8 in flight
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("axis", [0, 1])
+def test_face_thickness_of_few_layers_matches_the_oracle(gpu, n, axis):
+    print("[gpu case] face thickness", n, axis, flush=True)
+    rng = np.random.default_rng(n)
+    ny, nx = 37, 70
+    H = rng.uniform(5.0, 50.0, (ny, nx))
+    h = rng.dirichlet(np.ones(n), (ny, nx)).transpose(2, 0, 1) * H
+    h[rng.random(h.shape) < 0.02] = np.nan
+    act = rng.random((ny, nx)) > 0.1
+    got = ale.face_thickness_axis(_d(h), _d(H), _d(act), True, axis)
+    sw = (lambda x: x) if axis == 0 else (lambda x: np.ascontiguousarray(np.swapaxes(x, -1, -2)))
+    for g, w, nm in zip(got, R.face_transport_thickness(sw(h), sw(H), sw(act), True), ("q_pos", "q_neg")):
+        _bits(g, sw(w), nm)
