@@ -85,7 +85,9 @@ template <int AX>
 void launch_edges(const double* h, const uint8_t* act, double h_min, int n, int ny, int nx, double* lo, double* hi,
                   hipStream_t s) {
     Geo<AX> g{n, ny, nx};
-    const dim3 grid(blocks_for((long long)ny * nx), (unsigned)std::min((n + EDGE_LAYERS - 1) / EDGE_LAYERS, 65535));
+    const long long waves = ((long long)ny * nx + 63) / 64, slices = std::max(1LL, EDGE_WAVES / waves);
+    const int most = (n + EDGE_LAYERS - 1) / EDGE_LAYERS;
+    const dim3 grid(blocks_for((long long)ny * nx), (unsigned)std::min({slices, (long long)most, 65535LL}));
     k_ppm_edges<AX><<<grid, BS, 0, s>>>(h, act, h_min, g, lo, hi);
 }
 

@@ -259,11 +259,15 @@ __device__ __forceinline__ double ppm_slope(double hm1, double hc, double hp1, d
     return mw * me * m > 0.0 ? s : 0.0;
 }
 
-// one thread per cell (natural index j * nx + i) and every gridDim.y-th layer (about EDGE_LAYERS of them), which no
-// result of another layer enters: with all layers in one thread a small grid was one long chain of loads per wavefront
-// (198 x 159 x 50: 78-110 us a direction -> 21).  The thickness is read as the flux
+// one thread per cell (natural index j * nx + i) and every gridDim.y-th layer, which no result of another layer enters:
+// with all layers in one thread a small grid was one long chain of loads per wavefront (198 x 159 x 50: 78-110 us a
+// direction -> 21).  The layers are split only as far as that gives EDGE_WAVES wavefronts, and into slices of at least
+// EDGE_LAYERS layers: each slice reads the masks again and the layers in flight spread over memory (us, 1 / 2 / 4 / 13
+// slices: 384 x 384 x 50 110 / 78 / 68 / 62, 512 x 512 x 50 167 / 131 / 131 / 135, 724 x 724 x 50 258 / 258 / 259 / 271,
+// 1024 x 1024 x 50 504 / 510 / 512 / 528, 2000 x 2000 x 20 762 / 767 / 792 / 949).  The thickness is read as the flux
 // passes it: inactive cells 0, NaN 0.  Edges: lo = the low-index (west / south) edge, hi = the high one.
 constexpr int EDGE_LAYERS = 4;
+constexpr long long EDGE_WAVES = 24576;
 template <int AX>
 __global__ void k_ppm_edges(const double* __restrict__ h, const uint8_t* __restrict__ act, double h_min, Geo<AX> g,
                             double* __restrict__ e_lo, double* __restrict__ e_hi) {

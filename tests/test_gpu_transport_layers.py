@@ -213,3 +213,17 @@ def test_face_thickness_of_few_layers_matches_the_oracle(gpu, n, axis):
     sw = (lambda x: x) if axis == 0 else (lambda x: np.ascontiguousarray(np.swapaxes(x, -1, -2)))
     for g, w, nm in zip(got, R.face_transport_thickness(sw(h), sw(H), sw(act), True), ("q_pos", "q_neg")):
         _bits(g, sw(w), nm)
+
+
+# the edges' layers in one slice, in some and in slices of 4: planes on both sides of the line, ragged last slices
+@pytest.mark.parametrize("nx,ny,n", [(70, 37, 1), (70, 37, 9), (700, 760, 3), (512, 512, 21), (1030, 1020, 6)])
+@pytest.mark.parametrize("axis", [0, 1])
+def test_ppm_edges_of_every_slicing_match_the_oracle(gpu, nx, ny, n, axis):
+    print("[gpu case] edge slices", nx, ny, n, axis, flush=True)
+    rng = np.random.default_rng(n)
+    h = rng.uniform(0.0, 3.0, (n, ny, nx))
+    act = rng.random((ny, nx)) > 0.1
+    got = ale.ppm_edges_axis(_d(h), _d(act), axis)
+    sw = (lambda x: x) if axis == 0 else (lambda x: np.ascontiguousarray(np.swapaxes(x, -1, -2)))
+    for g, w, nm in zip(got, R.ppm_edges(sw(np.where(act, h, 0.0)), sw(act)), ("low", "high")):
+        _bits(g, sw(w), nm)
