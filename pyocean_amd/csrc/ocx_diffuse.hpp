@@ -20,14 +20,18 @@ namespace ocx {
 __device__ __forceinline__ double pymin(double a, double b) { return b < a ? b : a; }   // Python's min(a, b)
 
 // One thread per cell of layer k for every tracer of the stack (the per-layer fields are read once and serve all
-// tracers), block (64, DH_Y); rows are coalesced across lanes.  The blocks are a 1-D grid, x fastest, then y, then k,
-// remapped XCD-contiguously, so that the rows a block shares with those north and south of it come from one L2 (in
-// dispatch order neighbours sat on different XCDs and each fetched them from memory).  Where a row has a multiple of 8
-// blocks, dispatch order itself puts a block and its north and south neighbours on one XCD, and the 8 XCDs stay on
-// neighbouring rows: 1024 x 1024 x 50 x 10 3257 us, remapped 3375 (701 x 523 x 50 x 10 1242 and 1200).  Two tracers'
-// loads are in flight together, the volume's reciprocal is refined once for all tracers (qdiv_r gives the IEEE
-// quotient), and a T that is Tw is not read twice.  Bound by memory (20 B a tracer-cell, 3.5 TB/s): 701 x 523 x 50 x
-// 10 1186 us -> 1040, 384 x 384 x 50 x 10 449 -> 408; blocks of 8 or 16 rows 1048 and 1052.
+// tracers), block (64, DH_Y); rows are coalesced across lanes.  Two tracers' loads are in flight together, the volume's
+// reciprocal is refined once for all tracers (qdiv_r gives the IEEE quotient), and a T that is Tw is not read twice.
+//
+// The blocks are one range, x fastest, then y, then k.  In dispatch order neighbours sit on different XCDs, which share
+// the lines at a block's sides through memory: with rows that do not begin on a 64-byte line every block has such lines
+// and the XCD-contiguous order wins, and so it does where a row is one block and its neighbours north and south are the
+// next ones; elsewhere dispatch order is the better one, as it keeps the 8 XCDs on neighbouring rows (us, dispatch /
+// XCD-contiguous, T that is not Tw: 701 x 523 x 50 x 10 1252 / 1183, 333 x 500 x 30 x 8 306 / 292, 850 719 / 693, 1100 897
+// / 882, 700 551 / 558; 384 x 384 x 50 x 10 452 / 461, 768 x 768 x 50 x 10 1829 / 1870, 1024 x 1024 x 50 x 10 3243 / 3372,
+// 1040 x 500 x 30 x 8 811 / 851, 576 457 / 448; 64 x 500 x 30 x 8 43 / 35, 64 x 2048 x 50 x 10 399 / 407).  Bound by
+// memory, 20 B a tracer-cell (T that is Tw): 701 x 523 x 50 x 10 1022 us, 3.6 TB/s, against 1158 with one tracer in flight
+// and dispatch order; blocks of 8 or 16 rows 1 % slower.
 constexpr int DH_Y = 4;
 template <bool SAME>
 __global__ __launch_bounds__(64 * DH_Y) void k_diffuse_h(const double* __restrict__ T, const double* __restrict__ Tw,
@@ -38,7 +42,7 @@ __global__ __launch_bounds__(64 * DH_Y) void k_diffuse_h(const double* __restric
                                                    double kh, double dt, double* __restrict__ out) {
     const int gx = (nx + 63) / 64, gy = (ny + DH_Y - 1) / DH_Y;
     long long L = block_id();
-    if (gx % 8 != 0) L += xcd_logical((long long)blockIdx.x, (long long)gridDim.x) - blockIdx.x;
+    if (gx == 1 || nx % 8 != 0) L += xcd_logical((long long)blockIdx.x, (long long)gridDim.x) - blockIdx.x;
     const int i = (int)(L % gx) * 64 + threadIdx.x;
     L /= gx;
     const int j = (int)(L % gy) * DH_Y + threadIdx.y, k = (int)(L / gy);

@@ -79,3 +79,10 @@ def test_diffusion_of_one_and_of_two_arrays_match_the_oracle(gpu, nx, ny, nz, nt
     a, b = d(T), d(T)
     for got in (ops.diffuse_h(a, a, *args), ops.diffuse_h(a, b, *args)):
         assert np.array_equal(got.cpu().numpy(), want)
+
+
+# both block orders of the along-layer diffusion: rows of one block, of whole lines and of broken ones
+@pytest.mark.parametrize("nx,ny,nz,nt", [(40, 37, 3, 2), (64, 50, 5, 3), (72, 33, 4, 3), (136, 21, 7, 1),
+                                         (333, 18, 3, 4), (384, 9, 5, 2)])
+def test_diffusion_in_both_block_orders_matches_the_oracle(gpu, nx, ny, nz, nt):
+    test_diffusion_of_one_and_of_two_arrays_match_the_oracle(gpu, nx, ny, nz, nt)
