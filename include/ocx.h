@@ -262,6 +262,13 @@ int ocx_batch_destroy(ocx_batch* batch);
  * of each call, one wavefront per workgroup).  Process-wide. */
 int ocx_set_tuning(int rows_per_chunk, int waves_per_group);
 
+/* Launch shapes chosen by the size of a call (host computations; OCX_E_ARG for a shape the calls refuse): the rows per
+ * chunk of an FCT step under the current tuning, and the layers of a column that a workgroup of the RK3 step, the pc
+ * corrector or the RHS marches with the faces of these flags (OCX_CENTRED also for the pc predictor); nz: the whole
+ * column. */
+int ocx_fct_rows(int nt, int nz, int ny, int nx);
+int ocx_rk_layers(int nt, int nz, int ny, int nx, unsigned flags);
+
 /* Per-kernel timing (no counterpart in the reference; for benchmarks): while enabled, every kernel launch of this
  * library is bracketed by a hipEvent pair on its stream.  ocx_profile_collect waits for the recorded events,
  * returns the number of distinct kernels and fills up to max_kernels entries (static name strings, total

@@ -85,6 +85,8 @@ SIGNATURES = {
     "ocx_batch_graph_step": (I, [P, I, P]),
     "ocx_batch_destroy": (I, [P]),
     "ocx_set_tuning": (I, [I, I]),
+    "ocx_fct_rows": (I, [I, I, I, I]),
+    "ocx_rk_layers": (I, [I, I, I, I, U]),
     "ocx_profile_enable": (I, [I]),
     "ocx_profile_collect": (I, [I, P, P, P]),
 }

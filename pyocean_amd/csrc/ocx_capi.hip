@@ -57,9 +57,10 @@ long long rk_blocks(int nt, int ny, int nx, int tx) {
 // face) costs about 1.5 layers, and a launch takes as many rounds as its blocks need on the resident slots (3 blocks a
 // compute unit with the WENO faces, 4 with the cheaper ones), so the column is cut into the number of pieces that makes
 // rounds x (layers + 1.5) the least, if that is a tenth less than for the whole column; pieces beyond 64, or launches
-// beyond 2^24 blocks, never gain.  Whole column -> cut (us per step): RK3 128 x 128 x 20 x 2 tracers 285 -> 112 (4
-// layers; 2 layers 114, 10 layers 156), 198 x 159 x 50 x 1 717 -> 221 (5); 352 x 560 x 50 x 4 stays whole (3281,
-// pieces of 25 layers 3348), as does 1024 x 1024 x 50 x 10; pc with UP3 faces 128 x 128 x 20 x 2 110 -> 38 (3; 2 layers 44, 5 layers 43), 300 x 250 x 30 x 4 346 -> 289 (10).
+// beyond 2^24 blocks, never gain.  Whole column -> cut (us per step, layers a piece in brackets): RK3 128 x 128 x 20 x
+// 2 tracers 291 -> 117 (4; 2 layers 112, 10 layers 159), 198 x 159 x 50 x 1 735 -> 240 (10; 5 layers 238, 3 layers 236,
+// 25 layers 451); 352 x 560 x 50 x 4 stays whole (3281, pieces of 25 layers 3348), as does 1024 x 1024 x 50 x 10; pc
+// with UP3 faces 128 x 128 x 20 x 2 112 -> 40 (3; 2 layers 44, 5 layers 43), 300 x 250 x 30 x 4 360 -> 300 (10).
 int rk_layers(long long tiles, int nz, int blocks_per_cu) {
     const long long slots = 256LL * blocks_per_cu;
     int best = nz;
@@ -74,6 +75,11 @@ int rk_layers(long long tiles, int nz, int blocks_per_cu) {
         }
     }
     return best;
+}
+
+template <int SCH>
+int rk_piece(int nt, int nz, int ny, int nx) {
+    return rk_layers(rk_blocks(nt, ny, nx, rk_tx<SCH>()), nz, SCH <= ocx::SCH_Z ? 3 : 4);
 }
 
 int check_shape(int nt, int nz, int ny, int nx) {
@@ -256,7 +262,7 @@ template <int STAGE, int SCH, bool VERT>
 void rk_launch(const RkArgs& a, dim3, hipStream_t s) {
     constexpr int tx = rk_tx<SCH>(), ty = 256 / tx;
     const long long tiles = rk_blocks(a.nt, a.ny, a.nx, tx);
-    const int kl = rk_layers(tiles, a.nz, SCH <= ocx::SCH_Z ? 3 : 4);
+    const int kl = rk_piece<SCH>(a.nt, a.nz, a.ny, a.nx);
     const long long nb = tiles * ((a.nz + kl - 1) / kl);
     // the cut kernel is one of its own: its extra face costs the uncut one 6 % (registers), so a cut has to gain 10 %
     auto* kern = kl < a.nz ? ocx::k_rk_stage<STAGE, SCH, VERT, true, tx, ty>
@@ -894,6 +900,17 @@ void batch_free(ocx_batch* b) {
 }  // namespace
 
 extern "C" {
+
+int ocx_fct_rows(int nt, int nz, int ny, int nx) {
+    OCX_TRY(check_shape(nt, nz, ny, nx));
+    return rows_per_chunk(nt, nz, ny, nx);
+}
+
+int ocx_rk_layers(int nt, int nz, int ny, int nx, unsigned flags) {
+    OCX_TRY(check_shape(nt, nz, ny, nx));
+    return flags & (ocx::UP3 | ocx::UP1 | ocx::CENTRED) ? rk_piece<ocx::SCH_UP3>(nt, nz, ny, nx)
+                                                        : rk_piece<ocx::SCH_Z>(nt, nz, ny, nx);
+}
 
 int ocx_set_tuning(int rows_per_chunk, int waves_per_group) {
     if (rows_per_chunk < 0 || rows_per_chunk > (1 << 20) || waves_per_group < 0 || waves_per_group > ocx::MAXW)

@@ -474,9 +474,9 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(OCX_RK_W
                                                      int flux_face_i, int nt, int n, int ny, int nx, int kl, double dt,
                                                      unsigned flags) {
     // One block marches one tile of one tracer up its layers - all of them, or with CUT kl of them (1-D grid of
-    // nt * gx * gy * ceil(n / kl) blocks, XCD-contiguous): each layer's x and y faces go through the LDS tile; each thread keeps its column's window
-    // c[k-2 .. k+3] in registers and forms the z face between layers k and k+1 once, carrying it as the next layer's
-    // bottom face.
+    // nt * gx * gy * ceil(n / kl) blocks, XCD-contiguous): each layer's x and y faces go through the LDS tile; each
+    // thread keeps its column's window c[k-2 .. k+3] in registers and forms the z face between layers k and k+1 once,
+    // carrying it as the next layer's bottom face.
     constexpr bool ZF = VERT || SCH >= SCH_UP3;
     constexpr int H = 3, LX = TX + 2 * H, LY = TY + 2 * H;
     __shared__ double sc[LY * LX];

@@ -44,3 +44,13 @@ def test_ppm_workspace_holds_the_history_of_one_bundle(nx, ny, columns):
         size = [int(L.ocx_ppm_transport_workspace_bytes(50, ny, nx, axis, m)) for m in (8, 20)]
         want = columns * cols * 8
         assert abs(size[1] - size[0] - want) <= 512
+
+
+def test_rows_and_layers_of_a_call():
+    L = _native.lib()
+    assert [L.ocx_fct_rows(nt, nz, ny, nx) for nx, ny, nz, nt in (BASIN, BAY, (352, 560, 50, 2), (701, 523, 30, 10),
+                                                                 (1024, 1024, 50, 10))] == [2, 4, 16, 32, 64]
+    assert [L.ocx_rk_layers(2, 20, 128, 128, f) for f in (0, 16, 64, 128, 256)] == [4, 4, 3, 3, 3]
+    assert L.ocx_rk_layers(10, 50, 1024, 1024, 0) == L.ocx_rk_layers(10, 50, 1024, 1024, 64) == 50
+    assert L.ocx_rk_layers(1, 5, 320, 330, 0) == 5
+    assert L.ocx_fct_rows(1, 0, 1, 1) == L.ocx_rk_layers(1, 1, 0, 1, 0) == _native.OCX_E_ARG
