@@ -4,6 +4,8 @@ that stay below that.
 """
 from __future__ import annotations
 
+import gc
+
 import pytest
 import torch
 
@@ -13,6 +15,8 @@ pytestmark = pytest.mark.gpu
 
 
 def _need_memory(gib):
+    gc.collect()
+    torch.cuda.empty_cache()                           # what earlier tests left with torch's allocator
     if torch.cuda.mem_get_info()[0] < gib << 30:
         pytest.skip(f"needs {gib} GiB of device memory")
 
