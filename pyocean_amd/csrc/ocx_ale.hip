@@ -136,7 +136,8 @@ int ppm_impl(const double* h, const double* ut, const double* L, const double* Q
     OCX_TRY(launch_check("ppm init"));
     for (int m = 0; m < std::min(max_iter, p.single); ++m) {
         ProfScope _ps("ppm_newton", s);
-        if (walk)
+        // (an iteration past PPM_SINGLE mostly finds nothing to do, and a quarter of the workgroups leave sooner)
+        if (walk || m >= PPM_SINGLE)
             k_ppm_walk<AX, false><<<wb, BS, 0, s>>>(p, m);
         else
             k_ppm_pass<AX, false><<<gb, 64 * PPM_W, 0, s>>>(p, m);
