@@ -6,8 +6,8 @@ holds ``waves_per_group`` wavefronts, one tracer each, over the same strip, chun
 per-cell fields (Qx, Qy, V0, V1, ok) through the L1/L2.  A launch shape is therefore
 
 * ``rows_per_chunk`` - the y extent of one work item (each chunk re-reads a 3-row halo at its ends, so longer
-  chunks move fewer bytes but give fewer work items to spread over 256 compute units); 0: the untuned shape, whose
-  rows the library chooses by the wavefronts of the call, timed once;
+  chunks move fewer bytes but give fewer work items to spread over 256 compute units); 0: rows that the
+  library chooses by the wavefronts of the call, as in the untuned shape;
 * ``waves_per_group`` - the lane width of a workgroup, 64 x {1, 2, 4} lanes;
 * ``groups_per_cu`` (batches only) - the persistent grid, in workgroups per compute unit.
 
@@ -44,9 +44,9 @@ class Shape:
     @property
     def tile(self) -> str:
         """The work item as (x lanes) x (y rows) x (layers)."""
-        if not self.rows_per_chunk:
+        if self == Shape(0, 0, 0):
             return "untuned"
-        return f"{64 * max(self.waves_per_group, 1)}x{self.rows_per_chunk}x1"
+        return f"{64 * self.waves_per_group}x{self.rows_per_chunk or 'auto'}x1"
 
 
 def cache_path() -> Path:
@@ -86,8 +86,9 @@ def cached(kind: str, precision: str, shapes) -> Shape | None:
 
 
 def _candidates(rows, *others):
-    """The launch shapes to time: the untuned one once where ``rows`` holds 0, and every combination of the rest."""
-    return [(0,) * (1 + len(others))] * (0 in rows) + list(itertools.product([r for r in rows if r], *others))
+    """The launch shapes to time: every combination, after the untuned shape where ``rows`` holds 0."""
+    rows = tuple(rows)
+    return [(0,) * (1 + len(others))] * (0 in rows) + list(itertools.product(rows, *others))
 
 
 def _time_ms(fn, reps: int, stream) -> float:

@@ -41,6 +41,7 @@ def test_the_untuned_shape_is_a_candidate_and_can_win(fake):
     assert (0, 0, 0) in autotune._candidates(autotune.BATCH_ROWS, autotune.WAVES, autotune.GROUPS)
     assert _tune() == (best, [])                                    # cached
     assert autotune._candidates((16, 64), (1, 2)) == [(16, 1), (16, 2), (64, 1), (64, 2)]
+    assert autotune._candidates(iter((0, 64)), (1, 2)) == [(0, 0), (0, 1), (0, 2), (64, 1), (64, 2)]
 
 
 def test_a_winner_of_older_rules_is_not_taken(fake):
